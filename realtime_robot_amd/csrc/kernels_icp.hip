@@ -37,9 +37,21 @@ namespace rtr {
 constexpr uint32_t kFinishedBit = 1u << 30;
 constexpr int kMaxSpins = 1 << 22;
 
-__device__ __forceinline__ uint32_t load_acquire(const uint32_t* p) {
-  return __hip_atomic_load(p, __ATOMIC_ACQUIRE, __HIP_MEMORY_SCOPE_AGENT);
+// Synchronisation between workgroups.  Everything one workgroup hands to
+// another travels through two words: a problem's done count (an item's
+// partial sums and seeds are complete) and its generation word (the next
+// transform is published).  Each is written with one agent-scope release, and
+// a reader polls it with relaxed loads and takes one acquire once it has seen
+// the value it needs.  A release writes the XCD's L2 back and an acquire
+// invalidates the CU's L1, so polling with acquire loads, as this kernel once
+// did, emptied the L1 under the gathers of every other workgroup of the CU
+// each time an idle one looked at the queue: 32 pairs x 8 starts 89.3 -> 59.0
+// ms a launch, the learned call of 256 pairs 20.7 -> 11.3 ms, 256 pairs from
+// the identity 67.6 -> 66.3 ms.
+__device__ __forceinline__ uint32_t load_relaxed(const uint32_t* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ void acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 __device__ __forceinline__ void store_release(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
 }
@@ -416,12 +428,10 @@ __device__ void solve_problem(const DevEngine& e, uint32_t p, const Problem& pr,
   __syncthreads();
   if (gaa) {
     if (tid < kAndersonStride) gaa[tid] = sh.aa[tid];
-    __threadfence();
     __syncthreads();
   }
   if (tid == 0) {
     const bool fin = sh.fin != 0;
-    __threadfence();
     store_release((uint32_t*)&e.st[p].gen, (uint32_t)(pass + 1) | (fin ? kFinishedBit : 0u));
     if (fin) atomicAdd(e.problems_done, 1u);
   }
@@ -774,16 +784,15 @@ __device__ void process_item(const DevEngine& e, int it, int pass, IcpShared<NS,
     double s = sh.red[0][tid];
     for (int ww = 1; ww < kWaves; ++ww) s += sh.red[ww][tid];
     e.partials[(size_t)it * NSUM_MAX + tid] = s;
-    __threadfence();
   }
   __syncthreads();
   if (tid == 0) {
-    const uint32_t prev = atomicAdd(&e.done[p], 1u);
+    const uint32_t prev = __hip_atomic_fetch_add(&e.done[p], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
     sh.last = (prev + 1u == done_through(e, pr, pass));
+    if (sh.last) acquire_agent();
   }
   __syncthreads();
   if (sh.last) {
-    __threadfence();
     solve_problem<MODE, NS, TileT>(e, p, pr, td, pass, sh);
   }
 }
@@ -810,8 +819,8 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
     // leave between passes, holding no claimed item, and one workgroup per CU
     // stays, so every remaining item is still claimed.
     if (tid == 0) {
-      const uint32_t done = load_acquire(e.problems_done);
-      sh.stop = (done >= (uint32_t)e.n_prob) || (load_acquire((const uint32_t*)e.error) != 0u) ||
+      const uint32_t done = load_relaxed(e.problems_done);
+      sh.stop = (done >= (uint32_t)e.n_prob) || (load_relaxed((const uint32_t*)e.error) != 0u) ||
                 ((int)blockIdx.x >= e.retire_from && done + e.retire_active >= (uint32_t)e.n_prob);
     }
     __syncthreads();
@@ -832,7 +841,7 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
           if (c < cnt) {
             it = (int)(qoff[x] + c);
             const uint32_t p = e.items[it].x;
-            if (load_acquire((const uint32_t*)&e.st[p].gen) & kFinishedBit) {
+            if (load_relaxed((const uint32_t*)&e.st[p].gen) & kFinishedBit) {
               // a finished problem: its remaining items of this pass (contiguous
               // in this queue) are skipped in one step, and the claim goes on
               const Problem& pr = e.probs[p];
@@ -848,13 +857,13 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
         if (it < e.n_items) {
           const uint32_t p = e.items[it].x;
           const uint32_t* word = (const uint32_t*)&e.st[p].gen;
-          uint32_t wv = load_acquire(word);
+          uint32_t wv = load_relaxed(word);
           int spins = 0;
           // bounded wait with backoff; the error flag (on its own cache line)
           // is polled every 256 rounds
           while (!(wv & kFinishedBit) && (int)wv < pass) {
             ++spins;
-            if (spins > kMaxSpins || ((spins & 255) == 0 && load_acquire((const uint32_t*)e.error) != 0u)) {
+            if (spins > kMaxSpins || ((spins & 255) == 0 && load_relaxed((const uint32_t*)e.error) != 0u)) {
               atomicOr(e.error, 1);
               break;
             }
@@ -862,10 +871,11 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
               __builtin_amdgcn_s_sleep(1);
             else
               __builtin_amdgcn_s_sleep(8);
-            wv = load_acquire(word);
+            wv = load_relaxed(word);
           }
           if (!(wv & kFinishedBit) && (int)wv == pass) {
             run = 1;
+            acquire_agent();
             tf_rows_f32(e.st[p].T, sh.m);
             sh.stride = e.st[p].stage ? e.prm.coarse_stride : 1;
             const TargetDesc& td = e.tgts[e.probs[p].tgt];
