@@ -326,15 +326,97 @@ RTR_HD void walk_far(const GridView& g, float qx, float qy, float qz, int cx, in
   }
 }
 
-// Shells k0 + 1, k0 + 2, ... once the box of radius k0 has been searched
-// (or is known to be empty), each preceded by the stopping test.
+// Largest x with x * x <= v up to rounding (an upper estimate is wanted: the
+// callers widen it).
+RTR_HD float sqrt_approx(float v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  return __builtin_amdgcn_sqrtf(v);
+#else
+  return sqrtf(v);
+#endif
+}
+
+// Every cell that can hold a point within B = min(vis.bound(), r2f) of the
+// query, B finite and shrinking as points are found: x-rows in the order of
+// their distance from the query's own row (the nearer of the next row above
+// and below, plane by plane), each cut to the cells the remaining distance
+// reaches and read as one contiguous range.  Once the nearest row left in a
+// plane, or the nearest plane left, is beyond B, so are all behind it.  D: no
+// cell within Chebyshev distance D - 1 of (cx, cy, cz) holds a point (the
+// distance field's value, or 0), so a row that stays inside that box is
+// passed over.
+//
+// The bound on a row or plane is slab_gap's (axis gaps shortened by g.margin),
+// and a row is kept while gy^2 + gz^2 <= 1.000004 B, which keeps everything
+// that lb2_of's comparison keeps.  Along x the reach w covers sqrt of what is
+// left of B with 1e-5 to spare (the device square root is good to an ulp) and
+// two margins, so a point's own cell index, computed by the same float
+// expression, lies in [xa, xb].
 template <class V>
-RTR_HD void walk_outer(const GridView& g, float qx, float qy, float qz, int cx, int cy, int cz,
-                       float r2f, V& vis, int k0 = 1) {
-  const int kmax = (g.dx > g.dy ? (g.dx > g.dz ? g.dx : g.dz) : (g.dy > g.dz ? g.dy : g.dz));
-  for (int k = k0; k <= kmax; ++k) {
-    if (ring_done(g, qx, qy, qz, cx, cy, cz, k, r2f, vis)) return;
-    walk_shell(g, qx, qy, qz, cx, cy, cz, k + 1, r2f, vis);
+RTR_HD void walk_ball(const GridView& g, float qx, float qy, float qz, int cx, int cy, int cz, int D, float r2f,
+                      V& vis) {
+  constexpr float kFar = 1.0e18f;  // beyond the grid: above any gap whose square B can reach
+  // gap to row (plane) i above or below the query's own
+  auto above = [&](float q, float o, int i, int n) {
+    const float d = ((o + (float)i * g.h) - q) - g.margin;
+    return i < n ? (d > 0.f ? d : 0.f) : kFar;
+  };
+  auto below = [&](float q, float o, int i) {
+    const float d = (q - (o + (float)(i + 1) * g.h)) - g.margin;
+    return i >= 0 ? (d > 0.f ? d : 0.f) : kFar;
+  };
+  const float gy0 = slab_gap(qy, g.oy, g.h, g.margin, cy, cy), gz0 = slab_gap(qz, g.oz, g.h, g.margin, cz, cz);
+  int y = cy, z = cz, yu = cy + 1, yd = cy - 1, zu = cz + 1, zd = cz - 1;
+  float gy2 = gy0 * gy0, gz2 = gz0 * gz0;
+  float gyu = above(qy, g.oy, yu, g.dy), gyd = below(qy, g.oy, yd);
+  float gzu = above(qz, g.oz, zu, g.dz), gzd = below(qz, g.oz, zd);
+  for (;;) {
+    float B = (vis.bound() < r2f ? vis.bound() : r2f) * 1.000004f;
+    const float rem = B - (gy2 + gz2);
+    if (rem >= 0.f) {
+      const float w = sqrt_approx(rem) * 1.00001f + 2.0f * g.margin;
+      float fa = ((qx - w) - g.ox) * g.inv_h, fb = ((qx + w) - g.ox) * g.inv_h;
+      fa = fminf(fmaxf(fa, 0.f), 1.0e9f);
+      fb = fminf(fmaxf(fb, -1.f), 1.0e9f);
+      const int xa = (int)fa;                       // fa >= 0: truncation is the floor
+      const int xb0 = (int)floorf(fb);
+      const int xb = xb0 < g.dx - 1 ? xb0 : g.dx - 1;
+      const int ay = y > cy ? y - cy : cy - y, az = z > cz ? z - cz : cz - z;
+      const bool empty = ay < D && az < D && xa > cx - D && xb < cx + D;
+      if (xa <= xb && !empty) {
+        const uint32_t row = ((uint32_t)z * g.dy + y) * g.dx;
+        vis.scan(g.cell_start[row + xa], g.cell_start[row + xb + 1]);
+        B = (vis.bound() < r2f ? vis.bound() : r2f) * 1.000004f;
+      }
+    }
+    const float gn = fminf(gyu, gyd);
+    if (gn * gn + gz2 <= B) {
+      gy2 = gn * gn;
+      if (gyu <= gyd) {
+        y = yu++;
+        gyu = above(qy, g.oy, yu, g.dy);
+      } else {
+        y = yd--;
+        gyd = below(qy, g.oy, yd);
+      }
+      continue;
+    }
+    const float gp = fminf(gzu, gzd);
+    if (!(gp * gp <= B)) return;
+    gz2 = gp * gp;
+    if (gzu <= gzd) {
+      z = zu++;
+      gzu = above(qz, g.oz, zu, g.dz);
+    } else {
+      z = zd--;
+      gzd = below(qz, g.oz, zd);
+    }
+    y = cy;
+    gy2 = gy0 * gy0;
+    yu = cy + 1;
+    yd = cy - 1;
+    gyu = above(qy, g.oy, yu, g.dy);
+    gyd = below(qy, g.oy, yd);
   }
 }
 
@@ -354,10 +436,11 @@ RTR_HD void dist_caps(float r_max, float h, float margin, int* skip_ring, int* d
   }
 }
 
-// Ring walk that first consults the cell's distance D (a lower bound on the
-// Chebyshev distance to the nearest occupied cell): D >= skip_ring means no
-// point within r_max; D >= 2 means the 3x3x3 block is empty and the walk
-// starts at shell D.
+// The ICP search of one query (k_icp's, on any visitor): the cell's distance D
+// (a lower bound on the Chebyshev distance to the nearest occupied cell) is
+// consulted first, D >= skip_ring means no point within r_max.  With a finite
+// bound, from the visitor's seed or from r2f, one walk over the ball's rows;
+// else rings, from shell D when D >= 2 shows the 3x3x3 block empty.
 template <class V>
 RTR_HD void ring_walk_dt(const GridView& g, const uint8_t* dist, int skip_ring, float qx, float qy,
                          float qz, float r2f, V& vis) {
@@ -365,6 +448,10 @@ RTR_HD void ring_walk_dt(const GridView& g, const uint8_t* dist, int skip_ring, 
   if (!query_cell(g, qx, qy, qz, cx, cy, cz)) return;
   const int D = dist[((uint32_t)cz * g.dy + cy) * g.dx + cx];
   if (D >= skip_ring) return;
+  if ((vis.bound() < r2f ? vis.bound() : r2f) < 1.0e30f) {
+    walk_ball(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
+    return;
+  }
   int k0 = 1;
   if (D >= 2)
     k0 = D - 1;

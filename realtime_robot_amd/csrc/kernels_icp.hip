@@ -18,7 +18,7 @@
 // on a finished problem skips that problem's remaining items of the pass.
 //
 // Two search variants: the throughput variant (4 gathers in flight per lane,
-// 3 waves/SIMD) classifies an item's queries first and walks them from a
+// 3 or 4 waves/SIMD) classifies an item's queries first and walks them from a
 // compacted list grouped by distance-field class; the latency variant (8
 // gathers in flight, 2 waves/SIMD) walks each 64-query round directly.  With
 // Anderson acceleration on, the solving workgroup also extrapolates the next
@@ -214,42 +214,37 @@ struct GlobalVis {
     key = kNoKey;
     where = 0u;
   }
-  __device__ __forceinline__ void take(const float4& t, uint32_t j) {
-    const uint64_t k = nn_key(d2_f32(qx, qy, qz, t.x, t.y, t.z), __float_as_int(t.w));
-    if (k < key) {
-      key = k;
-      where = j | 0x80000000u;
-    }
-  }
   // D (4 or 8) independent loads in flight per step: the gathers are
   // latency-bound, and the deeper variant needs the registers of a kernel
-  // that runs 2 waves per SIMD
-  // (a walking pointer: one address per group, the loads at immediate offsets)
+  // that runs 2 waves per SIMD.  A range's last step loads its last point
+  // again in place of the missing ones (the same key twice changes nothing),
+  // so a short range costs one round of loads, not one per point.  A step
+  // whose smallest distance exceeds the best so far, most of them once the
+  // walk is seeded, ends there; else its points' keys are compared.
   __device__ __forceinline__ void scan(uint32_t b, uint32_t e) {
-    uint32_t j = b;
-    const float4* q = pts + b;
-    if (D == 8) {
-      for (; j + 8 <= e; j += 8, q += 8) {
-        const float4 t0 = q[0], t1 = q[1], t2 = q[2], t3 = q[3];
-        const float4 t4 = q[4], t5 = q[5], t6 = q[6], t7 = q[7];
-        take(t0, j);
-        take(t1, j + 1);
-        take(t2, j + 2);
-        take(t3, j + 3);
-        take(t4, j + 4);
-        take(t5, j + 5);
-        take(t6, j + 6);
-        take(t7, j + 7);
+    if (b >= e) return;
+    const uint32_t last = e - 1;
+    for (uint32_t j = b; j < e; j += D) {
+      float4 t[D];
+#pragma unroll
+      for (int u = 0; u < D; ++u) t[u] = pts[min(j + u, last)];
+      float d[D];
+#pragma unroll
+      for (int u = 0; u < D; ++u) d[u] = d2_f32(qx, qy, qz, t[u].x, t[u].y, t[u].z);
+      float m = d[0];
+#pragma unroll
+      for (int u = 1; u < D; ++u) m = fminf(m, d[u]);
+      if (m <= key_d2(key)) {
+#pragma unroll
+        for (int u = 0; u < D; ++u) {
+          const uint64_t k = nn_key(d[u], __float_as_int(t[u].w));
+          if (k < key) {
+            key = k;
+            where = min(j + u, last) | 0x80000000u;
+          }
+        }
       }
     }
-    for (; j + 4 <= e; j += 4, q += 4) {
-      const float4 t0 = q[0], t1 = q[1], t2 = q[2], t3 = q[3];
-      take(t0, j);
-      take(t1, j + 1);
-      take(t2, j + 2);
-      take(t3, j + 3);
-    }
-    for (; j < e; ++j, ++q) take(*q, j);
   }
   __device__ __forceinline__ float bound() const { return key_d2(key); }
   // Start from target point s (cell-sorted slot): its distance is an upper
@@ -312,6 +307,33 @@ __device__ __forceinline__ void walk_block_global(const GridView& g, float qx, f
     if (row_skip(lb2, vis.bound(), r2f)) continue;
     vis.scan(rb[k], re[k]);
   }
+}
+
+// The nearest target point of a query, from global memory.  With a finite
+// bound (a seed, or a bounded correspondence distance) one walk over the rows
+// that the bound's ball meets; without one, rings around the query until
+// something is found.  D: the distance field's value of the query's cell.
+//
+// What bounds it: lanes of a wave walk in lockstep, each step two dependent
+// gathers (a row's cell bounds, then its points), and VALU issue about 40 % of
+// the cycles.  The shell-by-shell walk tested every row of every shell,
+// (2k + 1)^2 of them, to find the few a seeded query needs; the ball's rows
+// need no test beyond the first one out of reach on each side.  256 pairs from
+// the identity 66.3 -> 50.0 ms, 32 pairs x 8 starts 59 -> 31-35 ms, one 10k x
+// 20k pair 3.2 -> 2.2 ms, the learned call of 256 pairs 11.3 -> 9.6 ms
+// (identical results).  Measured and left out: two or four rows' bounds
+// gathered together and their points searched as one list (47.9-48.8 ms for
+// the 256 pairs, 38-50 ms for the 32 x 8: the bound then shrinks a step late),
+// and the lanes grouped by the seed's distance in cells instead of by D (52 ms).
+template <int DEPTH>
+__device__ __forceinline__ void search_global(const GridView& g, float qx, float qy, float qz, int cx, int cy, int cz,
+                                              int D, float r2f, GlobalVis<DEPTH>& vis) {
+  if (fminf(vis.bound(), r2f) < 1.0e30f) {
+    walk_ball(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
+    return;
+  }
+  if (D < 2) walk_block_global(g, qx, qy, qz, cx, cy, cz, r2f, vis);
+  walk_far(g, qx, qy, qz, cx, cy, cz, r2f, vis, D >= 2 ? D - 1 : 1);
 }
 
 template <class TileT>
@@ -602,8 +624,7 @@ __device__ void process_item(const DevEngine& e, int it, int pass, IcpShared<NS,
           vis.init(g.pts, qx, qy, qz);
           const uint32_t s0 = sh.qseed[o];
           if (s0 - g.pt_lo < g.n_pts) vis.seed(s0);
-          if (D < 2) walk_block_global(g, qx, qy, qz, cx, cy, cz, r2f, vis);
-          walk_far(g, qx, qy, qz, cx, cy, cz, r2f, vis, D >= 2 ? D - 1 : 1);
+          search_global(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
           // a seed that is still the nearest neighbour is not written again
           // (most queries of a converging problem keep theirs)
           if (seeds && vis.key != kNoKey && (vis.where & 0x7fffffffu) != s0) seeds[chunk + o] = vis.where & 0x7fffffffu;
@@ -654,8 +675,9 @@ __device__ void process_item(const DevEngine& e, int it, int pass, IcpShared<NS,
     // distance field: cells within D - 1 rings of the query's cell are empty
     bool blk = act;  // the lane walks its 3x3x3 block
     int k0 = 1;      // box radius searched (or known empty) before the outer walk
+    int D = 0;
     if (act && e.cell_dist) {
-      const int D = e.cell_dist[td.cell_off + ((uint32_t)cz * g.dy + cy) * g.dx + cx];
+      D = e.cell_dist[td.cell_off + ((uint32_t)cz * g.dy + cy) * g.dx + cx];
       if (D >= td.skip_ring) {
         act = false;  // every target point is farther than r_max
         blk = false;
@@ -712,7 +734,9 @@ __device__ void process_item(const DevEngine& e, int it, int pass, IcpShared<NS,
       }
     }
     if (act) {
-      if (!blk) {
+      if (!TILE) {
+        search_global(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
+      } else if (!blk) {
         // block known empty: only the outer rings
       } else if (staged) {
         const int xlo = max(cx - 1, 0) - X0;
@@ -753,7 +777,7 @@ __device__ void process_item(const DevEngine& e, int it, int pass, IcpShared<NS,
       } else {
         walk_block_global(g, qx, qy, qz, cx, cy, cz, r2f, vis);
       }
-      walk_far(g, qx, qy, qz, cx, cy, cz, r2f, vis, k0);
+      if (TILE) walk_far(g, qx, qy, qz, cx, cy, cz, r2f, vis, k0);
       if (seeds && vis.key != kNoKey && (vis.where & 0x7fffffffu) != s0) seeds[j] = vis.where & 0x7fffffffu;
       if (key_d2(vis.key) <= r2f) {
         float4 c;

@@ -127,6 +127,14 @@ int rtr_selfcheck_nn_stats(const float* tgt, size_t nt, const float* q, size_t n
     v.best.key = ~0ull;
     v.best.tx = v.best.ty = v.best.tz = 0.f;
     v.best.slot = 0xffffffffu;
+    // every other query starts from a seed, some point of the target, as the
+    // kernel's queries start from their last nearest neighbour
+    int cx, cy, cz;
+    if ((i & 1) && query_cell(g, v.qx, v.qy, v.qz, cx, cy, cz)) {
+      const uint32_t s0 = (uint32_t)((i * 2654435761ull) % nv);
+      v.scan(s0, s0 + 1);
+      v.ranges = v.cands = 0;
+    }
     ring_walk_dt(g, da.data(), skip_ring, v.qx, v.qy, v.qz, r2f, v);
     NNBest b = v.best;
     if (b.key != ~0ull && !(key_d2(b.key) <= r2f)) b.key = ~0ull;

@@ -163,6 +163,36 @@ def test_host_grid_search_on_surfaces():
             assert np.array_equal(i1, i2) and np.array_equal(d1, d2)
 
 
+@pytest.mark.parametrize("shape", ["lattice", "plane", "line", "one_cell", "far_origin", "single_point"])
+@pytest.mark.parametrize("rmax", [0.0101, 0.05, 0.7, None])
+def test_host_ball_walk_matches_brute_force(shape, rmax):
+    """The bounded walk (seeded and not) where its row and cell limits can go
+    wrong: points and queries on cell faces, grids one cell thick, queries far
+    outside on every side, distances equal to the bound, coordinates whose
+    rounding is the size of the margin."""
+    rng = np.random.default_rng(7)
+    g = np.arange(13, dtype=np.float32) * np.float32(0.05)
+    t = np.stack(np.meshgrid(g, g, g[:7], indexing="ij"), -1).reshape(-1, 3)
+    if shape == "plane":
+        t = t * np.float32([1, 1, 0])
+    elif shape == "line":
+        t = t * np.float32([0, 1, 0])
+    elif shape == "one_cell":
+        t = t * np.float32(0.01)
+    elif shape == "far_origin":
+        t = t + np.float32([400.0, -300.0, 250.0])
+    elif shape == "single_point":
+        t = t[5:6]
+    t = t.astype(np.float32)
+    lo, hi = t.min(0), t.max(0)
+    q = rng.uniform(lo - 0.4, hi + 0.4, (700, 3)).astype(np.float32)
+    q = np.concatenate([q, t[::5], t[::7] + np.float32([0.025, 0, 0]), t[::11] + np.float32([0, 0.05, -0.05])])
+    for cell in (0.0125, 0.05, 0.31):
+        i1, d1 = R.selfcheck_nn(t, q.astype(np.float32), cell, 1e30 if rmax is None else rmax)
+        i2, d2 = oracle.nn_brute(q.astype(np.float32), t, rmax)
+        assert np.array_equal(i1, i2) and np.array_equal(d1, d2)
+
+
 def test_host_solver_matches_oracle():
     from scipy.spatial.transform import Rotation
     rng = np.random.default_rng(4)
