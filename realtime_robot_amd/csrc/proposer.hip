@@ -11,6 +11,7 @@
 // function.h:35-109): both produce the initial pose that ICP refines.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <cmath>
 #include <cstdio>
@@ -35,12 +36,15 @@ __host__ __device__ __forceinline__ uint16_t f2bf(float f) {
   const uint32_t r = 0x7fffu + ((u >> 16) & 1u);
   return (uint16_t)((u + r) >> 16);
 }
+__host__ __device__ __forceinline__ float as_float(float v) { return v; }
 __host__ __device__ __forceinline__ float bf2f(uint16_t b) {
   const uint32_t u = (uint32_t)b << 16;
   float f;
   memcpy(&f, &u, 4);
   return f;
 }
+
+__host__ __device__ __forceinline__ float as_float(uint16_t b) { return bf2f(b); }
 
 constexpr int kP = 1024;      // points per cloud after FPS
 constexpr int kC0 = 16;       // input channels (xyz padded to the MFMA K granularity)
@@ -184,15 +188,25 @@ static void gemm(hipStream_t s, const uint16_t* A, int lda, int ta, const uint16
 }
 
 // ---------------------------------------------------------------------------
-// Fused point MLP + max-pool (inference)
+// Fused point MLP + max-pool
 //
 // Rows of a cloud go through 16 -> 64 -> 128 -> 256 with bias + ReLU +
 // BF16 rounding after every layer and only the per-channel maxima leave the
-// chip.  Each layer is the same sequence of v_mfma_f32_32x32x8bf16_1k steps
-// (k ascending) as k_gemm_bf16 and rounds where the layer-by-layer path
-// stores BF16, so the pooled features are bit-identical to it.  The
-// transposed weights sit in LDS for the workgroup's lifetime; each wave owns
-// a 32-row activation tile in LDS; workgroups stride over clouds.
+// chip (with ARG their rows too, for the backward, which recomputes the few
+// rows it needs).  Each layer is the same sequence of
+// v_mfma_f32_32x32x8bf16_1k steps (k ascending) as k_gemm_bf16 and rounds
+// where the layer-by-layer path stores BF16, so the pooled features are
+// bit-identical to it; of the first layer's two steps the second multiplies
+// channels 8-15, all zero, and is left out.  The transposed weights sit in LDS
+// for the workgroup's lifetime; each wave owns a 32-row activation tile in
+// LDS; workgroups stride over clouds.
+//
+// The points are read as they are (FP32 xyz, turned by a hypothesis' rotation
+// where there is one) and the features go out as the head's BF16 input rows:
+// no packed copy of the points (16 channels, 13 of them zero) and no
+// concatenation pass (118 and 127 us of a call on 256 pairs x 8 hypotheses).
+// With ARG 93 us for 512 clouds; the three products, the kept activations and
+// the pooling pass it replaces in training took 1.7 ms.
 // ---------------------------------------------------------------------------
 constexpr int kFWaves = 8;
 constexpr int kFThreads = kFWaves * 64;
@@ -204,7 +218,7 @@ struct FusedShared {
   uint16_t w3t[kC3][kC2 + kFPad];
   uint16_t act[kFWaves][32][kC2 + kFPad];
   float b1[kC1], b2[kC2], b3[kC3];
-  uint32_t cmax[kC3];
+  int cmax[kC3];
 };
 
 __device__ __forceinline__ bf16x4 lds4(const uint16_t* p) { return *reinterpret_cast<const bf16x4*>(p); }
@@ -214,6 +228,34 @@ __device__ __forceinline__ bf16x4 lds4(const uint16_t* p) { return *reinterpret_
 // to 0 first
 __device__ __forceinline__ uint16_t bf16_relu(float v) {
   return __builtin_bit_cast(uint16_t, (__bf16)(v > 0.f ? v : 0.f));
+}
+
+// two of them, the first in the low half
+__device__ __forceinline__ uint32_t bf16_pair(float a, float b) {
+  typedef float f32x2 __attribute__((ext_vector_type(2)));
+  typedef __bf16 bf16x2 __attribute__((ext_vector_type(2)));
+  const f32x2 v = {a, b};
+  return __builtin_bit_cast(uint32_t, __builtin_convertvector(v, bf16x2));
+}
+
+// A point as the first layer's A operand (channels 0-2 and a zero), turned by
+// the row-major Q when asked.
+__device__ __forceinline__ bf16x4 point_operand(const float* q, const float* Q, bool turned) {
+  float v[3] = {q[0], q[1], q[2]};
+  if (turned) {
+    float u[3];
+#pragma unroll
+    for (int c = 0; c < 3; ++c) {
+      u[c] = Q[3 * c] * v[0];
+      u[c] = u[c] + Q[3 * c + 1] * v[1];
+      u[c] = u[c] + Q[3 * c + 2] * v[2];
+    }
+    v[0] = u[0];
+    v[1] = u[1];
+    v[2] = u[2];
+  }
+  const bf16x4 a = {(short)f2bf(v[0]), (short)f2bf(v[1]), (short)f2bf(v[2]), 0};
+  return a;
 }
 
 // The hardware conversion against f2bf over every non-NaN float: 16 bit
@@ -233,8 +275,20 @@ __global__ __launch_bounds__(256) void k_bf16_check(unsigned long long* bad) {
 // acc row of register j for this lane (32x32 MFMA output layout)
 __device__ __forceinline__ int mfma_row(int lane, int j) { return (j >> 2) * 8 + (lane >> 5) * 4 + (j & 3); }
 
-__global__ __launch_bounds__(kFThreads) void k_mlp_pool(const uint16_t* x0, int n_clouds, const uint16_t* wb,
-                                                       const float* w, ParamLayout L, float* G) {
+// The clouds of one pass.  k == 0: FPS clouds in their order (source 0, target
+// 0, source 1, ...), features to F row c / 2, half c % 2.  k > 0: the n
+// sources turned by rots[0], by rots[1], ..., then the n targets; source cloud
+// r = j * n + p fills the first half of F row r, target cloud p the second
+// half of the rows p, n + p, ...
+struct CloudSet {
+  const float* pts;   // FPS clouds as src0, tgt0, src1, ...: kP x 3 each
+  const float* rots;  // k row-major 3x3
+  int n, k;
+};
+
+template <bool ARG>
+__global__ __launch_bounds__(kFThreads) void k_mlp_pool(CloudSet cs, int n_clouds, const uint16_t* wb, const float* w,
+                                                       ParamLayout L, uint16_t* F, float* G, int32_t* arg) {
   extern __shared__ __align__(16) unsigned char smem_raw[];
   FusedShared& sh = *reinterpret_cast<FusedShared*>(smem_raw);
   const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
@@ -248,23 +302,32 @@ __global__ __launch_bounds__(kFThreads) void k_mlp_pool(const uint16_t* x0, int 
   uint16_t(*act)[kC2 + kFPad] = sh.act[wv];
   const int lr = lane & 31, kh = (lane >> 5) * 4;
   for (int c = blockIdx.x; c < n_clouds; c += gridDim.x) {
-    for (int i = tid; i < kC3; i += kFThreads) sh.cmax[i] = 0u;
+    for (int i = tid; i < kC3; i += kFThreads) sh.cmax[i] = 0;
     __syncthreads();
+    const int tgt0 = cs.k * cs.n;                     // first target cloud (k > 0)
+    const bool turned = cs.k > 0 && c < tgt0;
+    const int p = cs.k > 0 ? c % cs.n : 0;            // its pair
+    const float* const cp = cs.pts + (size_t)(cs.k > 0 ? 2 * p + (turned ? 0 : 1) : c) * kP * 3;
+    const float* const Q = turned ? cs.rots + 9 * (c / cs.n) : cs.rots;
+    // running maxima: the ReLU outputs, or with ARG the rounded output's bits
+    // over (kP - 1 - row), whose largest is the largest output's lowest row
     float vmax[kC3 / 32];
+    int kmax[kC3 / 32];
 #pragma unroll
-    for (int t = 0; t < kC3 / 32; ++t) vmax[t] = 0.f;
+    for (int t = 0; t < kC3 / 32; ++t) {
+      vmax[t] = 0.f;
+      kmax[t] = kP - 1;
+    }
     for (int r0 = wv * 32; r0 < kP; r0 += kFWaves * 32) {
-      const uint16_t* xr = x0 + ((size_t)c * kP + r0 + lr) * kC0;
-      // layer 1: K = 16 (two k-steps), N = 64 (two tiles)
-      const bf16x4 a0 = *reinterpret_cast<const bf16x4*>(xr + kh);
-      const bf16x4 a1 = *reinterpret_cast<const bf16x4*>(xr + 8 + kh);
+      // layer 1: K = 3 of a k-step's 8 (channels 3.. are zero), N = 64 (two tiles)
+      bf16x4 a0 = {0, 0, 0, 0};
+      if (kh == 0) a0 = point_operand(cp + 3 * (size_t)(r0 + lr), Q, turned);
 #pragma unroll
       for (int nt = 0; nt < kC1 / 32; ++nt) {
         f32x16 acc;
 #pragma unroll
         for (int j = 0; j < 16; ++j) acc[j] = 0.f;
         acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a0, lds4(&sh.w1t[nt * 32 + lr][kh]), acc, 0, 0, 0);
-        acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a1, lds4(&sh.w1t[nt * 32 + lr][8 + kh]), acc, 0, 0, 0);
         const int col = nt * 32 + lr;
 #pragma unroll
         for (int j = 0; j < 16; ++j) {
@@ -319,15 +382,29 @@ __global__ __launch_bounds__(kFThreads) void k_mlp_pool(const uint16_t* x0, int 
         // the pooled value is the BF16 rounding of the largest ReLU output:
         // rounding is monotone, so rounding the maximum once equals the
         // maximum of the rounded outputs; fmaxf(m, v) with m >= 0 is the
-        // ReLU (a NaN v leaves m, as ReLU maps NaN to 0)
+        // ReLU (a NaN v leaves m, as ReLU maps NaN to 0).  With ARG equal
+        // rounded outputs go to the lowest row, so every output is rounded;
+        // a -0 output is a negative key and leaves the +0 it starts from.
 #pragma unroll
         for (int t = 0; t < 4; ++t) {
           const int col = (half * 4 + t) * 32 + lr;
           const float b = sh.b3[col];
-          float m = vmax[half * 4 + t];
+          if (!ARG) {
+            float m = vmax[half * 4 + t];
 #pragma unroll
-          for (int j = 0; j < 16; ++j) m = fmaxf(m, acc[t][j] + b);
-          vmax[half * 4 + t] = m;
+            for (int j = 0; j < 16; ++j) m = fmaxf(m, acc[t][j] + b);
+            vmax[half * 4 + t] = m;
+          } else {
+            int m = kmax[half * 4 + t];
+#pragma unroll
+            for (int j = 0; j < 16; j += 2) {
+              const uint32_t pk = bf16_pair(fmaxf(acc[t][j] + b, 0.f), fmaxf(acc[t][j + 1] + b, 0.f));
+              const int rest = kP - 1 - r0 - mfma_row(lane, j);
+              m = max(m, (int)((pk << 16) | (uint32_t)rest));
+              m = max(m, (int)((pk & 0xffff0000u) | (uint32_t)(rest - 1)));
+            }
+            kmax[half * 4 + t] = m;
+          }
         }
       }
       __builtin_amdgcn_wave_barrier();  // act is rewritten by the next rows
@@ -335,13 +412,31 @@ __global__ __launch_bounds__(kFThreads) void k_mlp_pool(const uint16_t* x0, int 
     // lanes l and l + 32 hold different rows of the same channels
 #pragma unroll
     for (int t = 0; t < kC3 / 32; ++t) {
-      const float o = __shfl_xor(vmax[t], 32, 64);
-      const float mx = fmaxf(vmax[t], o);
-      const float m = bf2f(f2bf(mx > 0.f ? mx : 0.f));  // a -0 maximum becomes +0, as the ReLU gives
-      if (lane < 32) atomicMax(&sh.cmax[t * 32 + lane], __float_as_uint(m));  // m >= 0: bits order as floats
+      int key;
+      if (ARG) {
+        key = max(kmax[t], __shfl_xor(kmax[t], 32, 64));
+      } else {
+        const float o = __shfl_xor(vmax[t], 32, 64);
+        const float mx = fmaxf(vmax[t], o);
+        key = (int)((uint32_t)f2bf(mx > 0.f ? mx : 0.f) << 16);  // a -0 maximum becomes +0, as the ReLU gives
+      }
+      if (lane < 32) atomicMax(&sh.cmax[t * 32 + lane], key);  // key >= 0: bits order as floats
     }
     __syncthreads();
-    for (int i = tid; i < kC3; i += kFThreads) G[(size_t)c * kC3 + i] = __uint_as_float(sh.cmax[i]);
+    for (int i = tid; i < kC3; i += kFThreads) {
+      const uint32_t key = (uint32_t)sh.cmax[i];
+      const uint16_t f = (uint16_t)(key >> 16);
+      if (cs.k == 0)
+        F[(size_t)(c >> 1) * (2 * kC3) + (c & 1) * kC3 + i] = f;
+      else if (turned)
+        F[(size_t)c * (2 * kC3) + i] = f;
+      else
+        for (int j = 0; j < cs.k; ++j) F[((size_t)j * cs.n + p) * (2 * kC3) + kC3 + i] = f;
+      if (ARG) {
+        G[(size_t)c * kC3 + i] = bf2f(f);
+        arg[(size_t)c * kC3 + i] = kP - 1 - (int)(key & 0xffffu);
+      }
+    }
     __syncthreads();
   }
 }
@@ -425,7 +520,7 @@ __device__ __forceinline__ uint32_t fps_cell(float t) { return t >= 15.f ? 15u :
 
 __global__ __launch_bounds__(kFpsThreads, 4) void k_fps(const float* raw, const uint32_t* off, const uint32_t* cnt,
                                                      float* pts_out /* cloud * kP * 3 */,
-                                                     uint16_t* x0 /* rows of kC0 */, float* centroid /* cloud * 3 */,
+                                                     float* centroid /* cloud * 3 */,
                                                      int32_t* sel_out /* cloud*kP */) {
   const int c = blockIdx.x, tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const uint32_t n = cnt[c];
@@ -707,10 +802,6 @@ __global__ __launch_bounds__(kFpsThreads, 4) void k_fps(const float* raw, const 
     pts_out[3 * o + 2] = s_sel[s][2];
     if (sel_out) sel_out[o] = s_cur[s];
   }
-  for (int t = tid; t < kP * kC0; t += kFpsThreads) {
-    const int s = t / kC0, ch = t % kC0;
-    x0[(size_t)c * kP * kC0 + t] = f2bf(ch < 3 ? s_sel[s][ch] : 0.f);
-  }
 }
 
 // ---------------------------------------------------------------------------
@@ -751,12 +842,37 @@ __device__ __forceinline__ void cross3(const double* a, const double* b, double*
 }
 __device__ __forceinline__ double dot3(const double* a, const double* b) { return a[0] * b[0] + a[1] * b[1] + a[2] * b[2]; }
 
+// First and second moments of every pair's source points: sums of x, y, z, xx,
+// xy, xz, yy, yz, zz.  One wave per pair (one lane per pair, in k_head, walked
+// its 1024 points serially: 126 us for 256 pairs).
+__global__ __launch_bounds__(64) void k_moments(const float* pts /* cloud*kP*3 */, double* mom) {
+  const float* sp = pts + (size_t)(2 * blockIdx.x) * kP * 3;
+  double m[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
+  for (int i = threadIdx.x; i < kP; i += 64) {
+    const double x = sp[3 * i], y = sp[3 * i + 1], z = sp[3 * i + 2];
+    m[0] += x;
+    m[1] += y;
+    m[2] += z;
+    m[3] += x * x;
+    m[4] += x * y;
+    m[5] += x * z;
+    m[6] += y * y;
+    m[7] += y * z;
+    m[8] += z * z;
+  }
+#pragma unroll
+  for (int k = 0; k < 9; ++k) {
+    const double t = wave_sum_f64(m[k]);
+    if (threadIdx.x == 0) mom[9 * (size_t)blockIdx.x + k] = t;
+  }
+}
+
 // 6D -> rotation by Gram-Schmidt (columns b1, b2, b3 = b1 x b2), translation
 // o[6..8].  Loss per pair: mean over the source's FPS points s of
 // ||(R - R*) s + (t - t*)||^2 = tr(dR S dR^T) + 2 dt^T dR m + |dt|^2 with
 // S = mean s s^T, m = mean s.  Writes R, t (poses) and, when labels are
 // given, the loss and dL/dO.
-__global__ void k_head(const float* O, int n_pairs, const float* pts /* cloud*kP*3 */, const double* lab /* n*12 */,
+__global__ void k_head(const float* O, int n_pairs, const double* mom /* n*9 (k_moments) */, const double* lab /* n*12 */,
                        double* pose /* n*12 (R row-major, t) */, float* dO, float* loss) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
   if (p >= n_pairs) return;
@@ -780,17 +896,9 @@ __global__ void k_head(const float* O, int n_pairs, const float* pts /* cloud*kP
   for (int k = 0; k < 3; ++k) pose[(size_t)p * 12 + 9 + k] = t[k];
   if (!lab) return;
   // moments of the source FPS points (cloud 2p)
-  double S[9] = {0}, mm[3] = {0};
-  const float* sp = pts + (size_t)(2 * p) * kP * 3;
-  for (int i = 0; i < kP; ++i) {
-    const double s[3] = {sp[3 * i], sp[3 * i + 1], sp[3 * i + 2]};
-    for (int a = 0; a < 3; ++a) {
-      mm[a] += s[a];
-      for (int b = 0; b < 3; ++b) S[a * 3 + b] += s[a] * s[b];
-    }
-  }
-  for (int a = 0; a < 3; ++a) mm[a] /= kP;
-  for (int k = 0; k < 9; ++k) S[k] /= kP;
+  const double* q = mom + 9 * (size_t)p;
+  const double mm[3] = {q[0] / kP, q[1] / kP, q[2] / kP};
+  const double S[9] = {q[3] / kP, q[4] / kP, q[5] / kP, q[4] / kP, q[6] / kP, q[7] / kP, q[5] / kP, q[7] / kP, q[8] / kP};
   const double* L = lab + (size_t)p * 12;
   double dR[9], dt[3];
   for (int k = 0; k < 9; ++k) dR[k] = R[k] - L[k];
@@ -844,50 +952,283 @@ __global__ void k_relu_back(const float* dY, const uint16_t* Y, size_t n, uint16
     out[i] = bf2f(Y[i]) > 0.f ? f2bf(dY[i]) : (uint16_t)0;
 }
 
-// Max-pool + ReLU backward fused: the gradient of the pre-activation of
-// layer 3 is dG at each channel's argmax row when the pooled value is
-// positive (ReLU passes it), zero elsewhere; written as bf16.
-__global__ void k_pool_back(const float* dG /* cloud x C */, const int32_t* arg, const float* G, int C,
-                            size_t rows, uint16_t* out) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < rows * C; i += (size_t)gridDim.x * blockDim.x) {
-    const size_t row = i / C;
-    const int ch = (int)(i - row * C);
-    const size_t cl = row / kP;
-    const size_t gi = cl * C + ch;
-    const bool hit = arg[gi] == (int32_t)(row - cl * kP) && G[gi] > 0.f;
-    out[i] = hit ? f2bf(dG[gi]) : (uint16_t)0;
+// Column sums of a small matrix (the head's bias gradients): 64 columns per
+// workgroup, its 16 waves over the rows.
+template <class T>
+__global__ __launch_bounds__(1024) void k_colsum(const T* Y, int rows, int C, float* out) {
+  __shared__ float part[16][64];
+  const int lane = threadIdx.x & 63, w = threadIdx.x >> 6, ch = blockIdx.x * 64 + lane;
+  float s = 0.f;
+  if (ch < C)
+    for (int r = w; r < rows; r += 16) s += as_float(Y[(size_t)r * C + ch]);
+  part[w][lane] = s;
+  __syncthreads();
+  if (w == 0 && ch < C) {
+    for (int v = 1; v < 16; ++v) s += part[v][lane];
+    out[ch] = s;
   }
 }
 
-// dF (pairs x 512) -> dG (clouds x 256)
-__global__ void k_split(const float* dF, int n_pairs, float* dG) {
-  const int p = blockIdx.x, ch = threadIdx.x;
-  if (p >= n_pairs) return;
-  const float v = dF[(size_t)p * (2 * kC3) + ch];
-  if (ch < kC3)
-    dG[(size_t)(2 * p) * kC3 + ch] = v;
-  else
-    dG[(size_t)(2 * p + 1) * kC3 + (ch - kC3)] = v;
+// ---------------------------------------------------------------------------
+// Backward of the point MLP
+//
+// Max-pooling passes each channel's gradient to one row of its cloud, so of a
+// cloud's 1024 rows only the distinct argmax rows (at most 256, some 60-150 in
+// training) have any gradient at all: every other row adds zeros to the weight
+// and bias gradients.  One workgroup takes a cloud at a time: it lists those
+// rows, and for 32 of them at a time recomputes layers 1 and 2 (the forward's
+// own MFMA steps, so the same bits), and takes the gradient back through
+//   dA3: channel n's value at its row     (BF16, as stored by a dense pass)
+//   dW3, db3; dY2 = dA3 W3^T, dA2 = dY2 where Y2 > 0 (BF16)
+//   dW2, db2; dY1 = dA2 W2^T, dA1 = dY1 where Y1 > 0 (BF16)
+//   dW1, db1
+// with the weights in LDS (104 KB, one workgroup per CU) and every weight
+// gradient in registers until the workgroup's last cloud, then stored as one
+// partial per workgroup; k_sum_partials adds them in a fixed order.
+//
+// The dense pass this replaces ran the same products over all 1024 rows with
+// the activations (470 MB for 256 pairs) kept from the forward, an FP32 dY
+// written and read per layer, and column sums over 64 workgroups: about 10 ms
+// for 256 pairs, 7.7 of them the column sums, against 112 + 9 us here (the
+// whole gradient call 12.7 -> 0.75 ms).  What bounds this one: latency, two
+// clouds of 2-5 tiles per workgroup at one wave per SIMD.
+// ---------------------------------------------------------------------------
+constexpr int kBackThreads = 256;
+constexpr int kBackPad = 4;
+constexpr size_t kBackParams = (size_t)kC0 * kC1 + kC1 + (size_t)kC1 * kC2 + kC2 + (size_t)kC2 * kC3 + kC3;  // W1 .. b3
+
+struct BackShared {
+  uint16_t w1t[kC1][kC0 + kBackPad];  // layer 1, 2 forward: [out][in]
+  uint16_t w2t[kC2][kC1 + kBackPad];
+  uint16_t w2[kC1][kC2 + kBackPad];   // backward: [in][out]
+  uint16_t w3[kC2][kC3 + kBackPad];
+  float b1[kC1], b2[kC2];
+  // the tile: activations and gradients by row, and transposed ([channel][row])
+  uint16_t y1t[kC1][32 + kBackPad];
+  uint16_t y1[32][kC1 + kBackPad];
+  uint16_t y2[32][kC2 + kBackPad];    // Y2, then dA2
+  uint16_t da2t[kC2][32 + kBackPad];
+  float x[32][4];                     // the rows' points, rounded to BF16
+  // the cloud: active rows and each channel's place among them
+  uint32_t mask[kP / 32], pref[kP / 32];
+  uint16_t rows[kC3];
+  __align__(8) uint16_t val[kC3];     // dA3 of channel n at its row (BF16)
+  __align__(4) uint8_t slot[kC3];     // that row's place in rows
+  int n_rows;
+};
+
+__global__ __launch_bounds__(kBackThreads, 1) void k_mlp_back(const float* pts, int n_clouds, const uint16_t* wb,
+                                                           const float* w, ParamLayout L, const float* dF,
+                                                           const int32_t* arg, const float* G, float* partial) {
+  extern __shared__ __align__(16) unsigned char smem_raw[];
+  BackShared& sh = *reinterpret_cast<BackShared*>(smem_raw);
+  const int tid = threadIdx.x, lane = tid & 63, wv = tid >> 6;
+  const int lr = lane & 31, kh = (lane >> 5) * 4;
+  for (int i = tid; i < kC0 * kC1; i += kBackThreads) sh.w1t[i % kC1][i / kC1] = wb[L.W1 + i];
+  for (int i = tid; i < kC1 * kC2; i += kBackThreads) {
+    const uint16_t v = wb[L.W2 + i];
+    sh.w2t[i % kC2][i / kC2] = v;
+    sh.w2[i / kC2][i % kC2] = v;
+  }
+  for (int i = tid; i < kC2 * kC3; i += kBackThreads) sh.w3[i / kC3][i % kC3] = wb[L.W3 + i];
+  for (int i = tid; i < kC1; i += kBackThreads) sh.b1[i] = w[L.b1 + i];
+  for (int i = tid; i < kC2; i += kBackThreads) sh.b2[i] = w[L.b2 + i];
+  // gradients: thread n holds column n of W3 and b3[n]; wave v the columns
+  // 32 v .. of W2 and b2; waves 0 and 1 the columns 32 v .. of W1 and b1
+  float g3[kC2], gb3 = 0.f, g1[3] = {0.f, 0.f, 0.f}, gb1 = 0.f, gb2 = 0.f;
+  f32x16 g2[2];
+#pragma unroll
+  for (int k = 0; k < kC2; ++k) g3[k] = 0.f;
+#pragma unroll
+  for (int j = 0; j < 16; ++j) g2[0][j] = g2[1][j] = 0.f;
+  for (int c = blockIdx.x; c < n_clouds; c += gridDim.x) {
+    // ---- active rows of the cloud
+    __syncthreads();
+    if (tid < kP / 32) sh.mask[tid] = 0u;
+    __syncthreads();
+    const int row = arg[(size_t)c * kC3 + tid];
+    uint16_t v = 0;
+    if (G[(size_t)c * kC3 + tid] > 0.f) {
+      v = f2bf(dF[(size_t)(c >> 1) * (2 * kC3) + (c & 1) * kC3 + tid]);
+      atomicOr(&sh.mask[row >> 5], 1u << (row & 31));
+    }
+    sh.val[tid] = v;
+    gb3 += bf2f(v);
+    __syncthreads();
+    if (tid < 64) {
+      uint32_t n = tid < kP / 32 ? (uint32_t)__popc(sh.mask[tid]) : 0u, inc = n;
+#pragma unroll
+      for (int o = 1; o < 32; o <<= 1) {
+        const uint32_t u = __shfl_up(inc, o, 64);
+        if (lane >= o) inc += u;
+      }
+      if (tid < kP / 32) sh.pref[tid] = inc - n;
+      if (tid == kP / 32 - 1) sh.n_rows = (int)inc;
+    }
+    __syncthreads();
+    {
+      // (a channel without gradient has value 0: any slot serves it)
+      const uint32_t m = sh.mask[row >> 5], bit = 1u << (row & 31);
+      const uint32_t s = (m & bit) ? sh.pref[row >> 5] + (uint32_t)__popc(m & (bit - 1u)) : 0u;
+      sh.slot[tid] = (uint8_t)s;
+      if (m & bit) sh.rows[s] = (uint16_t)row;
+    }
+    __syncthreads();
+    const int n_rows = sh.n_rows;
+    const float* const cp = pts + (size_t)c * kP * 3;
+    for (int t0 = 0; t0 < n_rows; t0 += 32) {
+      // ---- layer 1 (waves 0 and 1, 32 channels each).  Places past the last
+      // active row repeat it: no channel names them, so their gradient is zero.
+      uint32_t on1 = 0u;  // Y1 > 0, one bit per accumulator register
+      if (wv < 2) {
+        bf16x4 a0 = {0, 0, 0, 0};
+        if (kh == 0) a0 = point_operand(cp + 3 * (size_t)sh.rows[min(t0 + lr, n_rows - 1)], nullptr, false);
+        if (wv == 0 && kh == 0) {
+          sh.x[lr][0] = bf2f((uint16_t)a0[0]);
+          sh.x[lr][1] = bf2f((uint16_t)a0[1]);
+          sh.x[lr][2] = bf2f((uint16_t)a0[2]);
+        }
+        f32x16 acc;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[j] = 0.f;
+        acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a0, lds4(&sh.w1t[wv * 32 + lr][kh]), acc, 0, 0, 0);
+        const int col = wv * 32 + lr;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const uint16_t y = bf16_relu(acc[j] + sh.b1[col]);
+          on1 |= (y != 0 ? 1u : 0u) << j;
+          sh.y1[mfma_row(lane, j)][col] = y;
+          sh.y1t[col][mfma_row(lane, j)] = y;
+        }
+      }
+      __syncthreads();
+      // ---- layer 2 (wave v: channels 32 v ..)
+      uint32_t on2 = 0u;
+      {
+        f32x16 acc;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) acc[j] = 0.f;
+#pragma unroll
+        for (int ks = 0; ks < kC1 / 8; ++ks)
+          acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(lds4(&sh.y1[lr][ks * 8 + kh]),
+                                                         lds4(&sh.w2t[wv * 32 + lr][ks * 8 + kh]), acc, 0, 0, 0);
+        const int col = wv * 32 + lr;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const uint16_t y = bf16_relu(acc[j] + sh.b2[col]);
+          on2 |= (y != 0 ? 1u : 0u) << j;
+          sh.y2[mfma_row(lane, j)][col] = y;
+        }
+      }
+      __syncthreads();
+      // ---- dW3: channel tid's row, when it is in this tile
+      {
+        const int s = (int)sh.slot[tid] - t0;
+        const float vf = bf2f(sh.val[tid]);
+        if (s >= 0 && s < 32 && vf != 0.f) {
+#pragma unroll
+          for (int k = 0; k < kC2; k += 4) {
+            const bf16x4 y = lds4(&sh.y2[s][k]);
+#pragma unroll
+            for (int u = 0; u < 4; ++u) g3[k + u] = fmaf(bf2f((uint16_t)y[u]), vf, g3[k + u]);
+          }
+        }
+      }
+      // ---- dY2 = dA3 W3^T: the A operand is built from the channels' slots
+      f32x16 acc;
+#pragma unroll
+      for (int j = 0; j < 16; ++j) acc[j] = 0.f;
+#pragma unroll 4
+      for (int ks = 0; ks < kC3 / 8; ++ks) {
+        const int n = ks * 8 + kh;
+        const uint32_t s4 = *reinterpret_cast<const uint32_t*>(&sh.slot[n]);
+        const bf16x4 v4 = lds4(&sh.val[n]);
+        bf16x4 a;
+#pragma unroll
+        for (int u = 0; u < 4; ++u) a[u] = (int)((s4 >> (8 * u)) & 0xffu) == t0 + lr ? v4[u] : (short)0;
+        acc = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(a, lds4(&sh.w3[wv * 32 + lr][n]), acc, 0, 0, 0);
+      }
+      __syncthreads();  // every read of Y2 is done: dA2 takes its place
+      {
+        const int col = wv * 32 + lr;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const uint16_t d = ((on2 >> j) & 1u) ? f2bf(acc[j]) : (uint16_t)0;
+          gb2 += bf2f(d);
+          sh.y2[mfma_row(lane, j)][col] = d;
+          sh.da2t[col][mfma_row(lane, j)] = d;
+        }
+      }
+      __syncthreads();
+      // ---- dW2 = Y1^T dA2 (wave v: columns 32 v .., both halves of the rows)
+#pragma unroll
+      for (int ks = 0; ks < 4; ++ks) {
+        const bf16x4 b = lds4(&sh.da2t[wv * 32 + lr][ks * 8 + kh]);
+#pragma unroll
+        for (int mt = 0; mt < 2; ++mt)
+          g2[mt] = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(lds4(&sh.y1t[mt * 32 + lr][ks * 8 + kh]), b, g2[mt], 0, 0, 0);
+      }
+      // ---- dY1 = dA2 W2^T, dA1, dW1, db1 (waves 0 and 1, 32 channels each)
+      if (wv < 2) {
+        f32x16 d1;
+#pragma unroll
+        for (int j = 0; j < 16; ++j) d1[j] = 0.f;
+#pragma unroll 4
+        for (int ks = 0; ks < kC2 / 8; ++ks)
+          d1 = __builtin_amdgcn_mfma_f32_32x32x8bf16_1k(lds4(&sh.y2[lr][ks * 8 + kh]),
+                                                        lds4(&sh.w2[wv * 32 + lr][ks * 8 + kh]), d1, 0, 0, 0);
+#pragma unroll
+        for (int j = 0; j < 16; ++j) {
+          const float d = ((on1 >> j) & 1u) ? bf2f(f2bf(d1[j])) : 0.f;
+          const float* xr = sh.x[mfma_row(lane, j)];
+          gb1 += d;
+          g1[0] = fmaf(xr[0], d, g1[0]);
+          g1[1] = fmaf(xr[1], d, g1[1]);
+          g1[2] = fmaf(xr[2], d, g1[2]);
+        }
+      }
+      __syncthreads();  // the next tile rewrites the activations
+    }
+  }
+  // ---- this workgroup's partial, in the parameters' layout
+  float* const o = partial + (size_t)blockIdx.x * kBackParams;
+  gb2 += __shfl_xor(gb2, 32, 64);
+  gb1 += __shfl_xor(gb1, 32, 64);
+#pragma unroll
+  for (int k = 0; k < 3; ++k) g1[k] += __shfl_xor(g1[k], 32, 64);
+  if (wv < 2 && lane < 32) {
+    const int col = wv * 32 + lane;
+    for (int r = 0; r < kC0; ++r) o[L.W1 + (size_t)r * kC1 + col] = r < 3 ? (r == 0 ? g1[0] : (r == 1 ? g1[1] : g1[2])) : 0.f;
+    o[L.b1 + col] = gb1;
+  }
+#pragma unroll
+  for (int mt = 0; mt < 2; ++mt)
+#pragma unroll
+    for (int j = 0; j < 16; ++j) o[L.W2 + (size_t)(mt * 32 + mfma_row(lane, j)) * kC2 + wv * 32 + lr] = g2[mt][j];
+  if (lane < 32) o[L.b2 + wv * 32 + lane] = gb2;
+#pragma unroll
+  for (int k = 0; k < kC2; ++k) o[L.W3 + (size_t)k * kC3 + tid] = g3[k];
+  o[L.b3 + tid] = gb3;
 }
 
-// column sums of a bf16 matrix (bias gradients), split over row chunks
-__global__ void k_colsum(const uint16_t* Y, size_t rows, int C, float* out) {
-  const int ch = threadIdx.x + blockIdx.y * blockDim.x;
-  if (ch >= C) return;
-  const size_t chunk = (rows + gridDim.x - 1) / gridDim.x;
-  const size_t r0 = blockIdx.x * chunk, r1 = min(rows, r0 + chunk);
+// g[i] = the sum of the workgroups' partials
+__global__ __launch_bounds__(256) void k_sum_partials(const float* partial, int n_parts, size_t n, float* g) {
+  const size_t i = (size_t)blockIdx.x * 64 + (threadIdx.x & 63);
+  const int w = threadIdx.x >> 6;
+  __shared__ float part[4][64];
   float s = 0.f;
-  for (size_t r = r0; r < r1; ++r) s += bf2f(Y[r * C + ch]);
-  atomicAdd(out + ch, s);
-}
-__global__ void k_colsum_f32(const float* Y, size_t rows, int C, float* out) {
-  const int ch = threadIdx.x + blockIdx.y * blockDim.x;
-  if (ch >= C) return;
-  const size_t chunk = (rows + gridDim.x - 1) / gridDim.x;
-  const size_t r0 = blockIdx.x * chunk, r1 = min(rows, r0 + chunk);
-  float s = 0.f;
-  for (size_t r = r0; r < r1; ++r) s += Y[r * C + ch];
-  atomicAdd(out + ch, s);
+  if (i < n) {
+    int b = w;
+    float t[4] = {0.f, 0.f, 0.f, 0.f};
+    for (; b + 12 < n_parts; b += 16)
+#pragma unroll
+      for (int u = 0; u < 4; ++u) t[u] += partial[(size_t)(b + 4 * u) * n + i];
+    for (; b < n_parts; b += 4) t[0] += partial[(size_t)b * n + i];
+    s = (t[0] + t[1]) + (t[2] + t[3]);
+  }
+  part[w][threadIdx.x & 63] = s;
+  __syncthreads();
+  if (w == 0 && i < n) g[i] = (part[0][threadIdx.x] + part[1][threadIdx.x]) + (part[2][threadIdx.x] + part[3][threadIdx.x]);
 }
 
 __global__ void k_to_bf16(const float* in, size_t n, uint16_t* out) {
@@ -994,11 +1335,6 @@ __global__ void k_pack_x0(const float* xyz, size_t rows, uint16_t* x0) {
   }
 }
 
-__global__ void k_zero(float* p, size_t n) {
-  for (size_t i = (size_t)blockIdx.x * blockDim.x + threadIdx.x; i < n; i += (size_t)gridDim.x * blockDim.x)
-    p[i] = 0.f;
-}
-
 // Adam (Kingma & Ba 2015) on the FP32 master weights; refreshes the BF16 copy.
 __global__ void k_adam(float* w, const float* g, float* m, float* v, size_t n, float lr, float b1, float b2,
                        float eps, float c1, float c2, uint16_t* wb) {
@@ -1031,7 +1367,7 @@ struct Proposer {
   DevBuf raw, roff, rcnt;           // resident raw clouds for proposals
   DevBuf pts, x0, cen, sel;         // FPS outputs
   DevBuf y1, y2, y3, G, arg, F, h1, O, pose, lab, dO, loss;
-  DevBuf dtmp, dbf, dG, dF, dH1, dH1b, dOb;
+  DevBuf mom, back, dF, dH1, dH1b, dOb;  // back: the point MLP's gradient partials, one per workgroup
   DevBuf rots, score;               // hypothesis rotations, candidate scores
   bool train_ready = false;
   int fused_blocks = 256;           // workgroups of the fused point MLP (one per CU)
@@ -1064,8 +1400,12 @@ struct Proposer {
     RTR_HIP(hipStreamCreateWithFlags(&stream, hipStreamNonBlocking));
     RTR_HIP(hipEventCreate(&ev0));
     RTR_HIP(hipEventCreate(&ev1));
-    RTR_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mlp_pool),
+    RTR_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mlp_pool<false>),
                                 hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(FusedShared)));
+    RTR_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mlp_pool<true>),
+                                hipFuncAttributeMaxDynamicSharedMemorySize, (int)sizeof(FusedShared)));
+    RTR_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(k_mlp_back), hipFuncAttributeMaxDynamicSharedMemorySize,
+                                (int)sizeof(BackShared)));
     int cus = 0;
     RTR_HIP(hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, device));
     fused_blocks = cus > 0 ? cus : 256;
@@ -1074,12 +1414,8 @@ struct Proposer {
     int rc = w.ensure(P * 4);
     if (!rc) rc = wb.ensure(P * 2);
     if (!rc) rc = pts.ensure(rows * 12);
-    if (!rc) rc = x0.ensure(rows * kC0 * 2);
     if (!rc) rc = cen.ensure(clouds * 12);
     if (!rc) rc = sel.ensure(rows * 4);
-    if (!rc) rc = y1.ensure(rows * kC1 * 2);
-    if (!rc) rc = y2.ensure(rows * kC2 * 2);
-    if (!rc) rc = y3.ensure(rows * kC3 * 2);
     if (!rc) rc = G.ensure(clouds * kC3 * 4);
     if (!rc) rc = arg.ensure(clouds * kC3 * 4);
     if (!rc) rc = F.ensure((size_t)maxp * 2 * kC3 * 2);
@@ -1096,7 +1432,7 @@ struct Proposer {
   int ensure_train() {
     if (train_ready) return RTR_OK;
     const size_t P = L.total;
-    const size_t clouds = 2 * (size_t)max_pairs, rows = clouds * kP;
+    const size_t clouds = 2 * (size_t)max_pairs;
     const size_t maxp = (size_t)max_pairs;
     int rc = g.ensure(P * 4);
     if (!rc) rc = m.ensure(P * 4);
@@ -1104,9 +1440,8 @@ struct Proposer {
     if (!rc) rc = lab.ensure(maxp * 12 * 8);
     if (!rc) rc = dO.ensure(maxp * kOut * 4);
     if (!rc) rc = loss.ensure(maxp * 4);
-    if (!rc) rc = dtmp.ensure(rows * kC3 * 4);
-    if (!rc) rc = dbf.ensure(rows * kC3 * 2);
-    if (!rc) rc = dG.ensure(clouds * kC3 * 4);
+    if (!rc) rc = mom.ensure(maxp * 9 * 8);
+    if (!rc) rc = back.ensure(std::min(clouds, (size_t)fused_blocks) * kBackParams * 4);
     if (!rc) rc = dF.ensure(maxp * 2 * kC3 * 4);
     if (!rc) rc = dH1.ensure(maxp * kH * 4);
     if (!rc) rc = dH1b.ensure(maxp * kH * 2);
@@ -1122,8 +1457,8 @@ struct Proposer {
     (void)hipSetDevice(device);
     if (stream) (void)hipStreamSynchronize(stream);
     DevBuf* all[] = {&w,  &wb,  &g,  &m,  &v,   &raw, &roff, &rcnt, &pts, &x0,  &cen,  &sel,  &y1,
-                     &y2, &y3,  &G,  &arg, &F,  &h1,  &O,    &pose, &lab, &dO,  &loss, &dtmp, &dbf,
-                     &dG, &dF,  &dH1, &dH1b, &dOb, &rots, &score};
+                     &y2, &y3,  &G,  &arg, &F,  &h1,  &O,    &pose, &lab, &dO,  &loss, &mom, &back,
+                     &dF,  &dH1, &dH1b, &dOb, &rots, &score};
     for (DevBuf* b : all) b->release();
     if (ev0) (void)hipEventDestroy(ev0);
     if (ev1) (void)hipEventDestroy(ev1);
@@ -1242,8 +1577,7 @@ struct Proposer {
   void enqueue_fps() {
     n_pairs = n_resident;
     hipLaunchKernelGGL(k_fps, dim3(2 * n_pairs), dim3(kFpsThreads), 0, stream, raw.as<float>(), roff.as<uint32_t>(),
-                       rcnt.as<uint32_t>(), pts.as<float>(), x0.as<uint16_t>(), cen.as<float>(),
-                       sel.as<int32_t>());
+                       rcnt.as<uint32_t>(), pts.as<float>(), cen.as<float>(), sel.as<int32_t>());
   }
 
   // FPS points given directly (training): centred xyz, n_pairs * 2 * kP
@@ -1256,23 +1590,33 @@ struct Proposer {
     n_pairs = np;
     const size_t rows = (size_t)2 * np * kP;
     RTR_HIP(hipMemcpyAsync(pts.p, xyz, rows * 12, hipMemcpyHostToDevice, stream));
-    hipLaunchKernelGGL(k_pack_x0, dim3(1024), dim3(256), 0, stream, pts.as<float>(), rows, x0.as<uint16_t>());
-    RTR_HIP(hipGetLastError());
     return RTR_OK;
   }
 
   const uint16_t* wbp(size_t off) const { return wb.as<uint16_t>() + off; }
   const float* wp(size_t off) const { return w.as<float>() + off; }
 
-  // pooled features G of C clouds from x0: fused for inference, layer by
-  // layer (activations and argmax kept for the backward) for training
-  void enqueue_point_mlp(int C, bool keep_activations) {
-    if (!keep_activations) {
-      const int grid = C < fused_blocks ? C : fused_blocks;
-      hipLaunchKernelGGL(k_mlp_pool, dim3(grid), dim3(kFThreads), sizeof(FusedShared), stream, x0.as<uint16_t>(), C,
-                         wb.as<uint16_t>(), w.as<float>(), L, G.as<float>());
-      return;
-    }
+  // The layer-by-layer path's activations (set_fused 0): never held otherwise.
+  int ensure_layers() {
+    const size_t rows = 2 * (size_t)max_pairs * kP;
+    int rc = x0.ensure(rows * kC0 * 2);
+    if (!rc) rc = y1.ensure(rows * kC1 * 2);
+    if (!rc) rc = y2.ensure(rows * kC2 * 2);
+    if (!rc) rc = y3.ensure(rows * kC3 * 2);
+    return rc;
+  }
+
+  // Head input rows F of the clouds: one fused pass; with backward the pooled
+  // maxima and their rows too.
+  void enqueue_point_mlp(const CloudSet& cs, int C, bool backward) {
+    const int grid = C < fused_blocks ? C : fused_blocks;
+    auto* kernel = backward ? k_mlp_pool<true> : k_mlp_pool<false>;
+    hipLaunchKernelGGL(kernel, dim3(grid), dim3(kFThreads), sizeof(FusedShared), stream, cs, C, wb.as<uint16_t>(),
+                       w.as<float>(), L, F.as<uint16_t>(), G.as<float>(), arg.as<int32_t>());
+  }
+
+  // The same features layer by layer, from the packed rows x0 (ensure_layers).
+  void enqueue_point_mlp_layers(int C) {
     const int rows = C * kP;
     gemm(stream, x0.as<uint16_t>(), kC0, 0, wbp(L.W1), kC1, 0, y1.p, kC1, rows, kC1, kC0, wp(L.b1), 1, 1);
     gemm(stream, y1.as<uint16_t>(), kC1, 0, wbp(L.W2), kC2, 0, y2.p, kC2, rows, kC2, kC1, wp(L.b2), 1, 1);
@@ -1281,76 +1625,74 @@ struct Proposer {
                        arg.as<int32_t>());
   }
 
-  void enqueue_forward(bool with_labels, bool keep_activations) {
+  int enqueue_forward(bool with_labels) {
     const int B = n_pairs, C = 2 * B;
-    enqueue_point_mlp(C, keep_activations);
-    hipLaunchKernelGGL(k_concat, dim3(B), dim3(2 * kC3), 0, stream, G.as<float>(), B, F.as<uint16_t>());
+    if (with_labels || !fused_off) {
+      enqueue_point_mlp(CloudSet{pts.as<float>(), nullptr, B, 0}, C, with_labels);
+    } else {
+      RTR_TRY(ensure_layers());
+      hipLaunchKernelGGL(k_pack_x0, dim3(1024), dim3(256), 0, stream, pts.as<float>(), (size_t)C * kP,
+                         x0.as<uint16_t>());
+      enqueue_point_mlp_layers(C);
+      hipLaunchKernelGGL(k_concat, dim3(B), dim3(2 * kC3), 0, stream, G.as<float>(), B, F.as<uint16_t>());
+    }
     gemm(stream, F.as<uint16_t>(), 2 * kC3, 0, wbp(L.W4), kH, 0, h1.p, kH, B, kH, 2 * kC3, wp(L.b4), 1, 1);
     gemm(stream, h1.as<uint16_t>(), kH, 0, wbp(L.W5), kOut, 0, O.p, kOut, B, kOut, kH, wp(L.b5), 0, 0);
-    hipLaunchKernelGGL(k_head, dim3((B + 63) / 64), dim3(64), 0, stream, O.as<float>(), B, pts.as<float>(),
+    if (with_labels)
+      hipLaunchKernelGGL(k_moments, dim3(B), dim3(64), 0, stream, pts.as<float>(), mom.as<double>());
+    hipLaunchKernelGGL(k_head, dim3((B + 63) / 64), dim3(64), 0, stream, O.as<float>(), B, mom.as<double>(),
                        with_labels ? lab.as<double>() : nullptr, pose.as<double>(), dO.as<float>(),
                        loss.as<float>());
+    return RTR_OK;
   }
 
   // Network over k hypotheses per resident pair (after enqueue_fps): point
   // MLP over (k+1)*n clouds, head over k*n rows, then candidate scores.
-  void enqueue_forward_multi(int k, float tau2) {
+  int enqueue_forward_multi(int k, float tau2) {
     const int n = n_pairs, C = (k + 1) * n, B = k * n;
-    hipLaunchKernelGGL(k_pack_multi, dim3(2048), dim3(256), 0, stream, pts.as<float>(), n, k, rots.as<float>(),
-                       x0.as<uint16_t>());
-    enqueue_point_mlp(C, fused_off);
-    hipLaunchKernelGGL(k_concat_multi, dim3(B), dim3(2 * kC3), 0, stream, G.as<float>(), n, k, F.as<uint16_t>());
+    if (!fused_off) {
+      enqueue_point_mlp(CloudSet{pts.as<float>(), rots.as<float>(), n, k}, C, false);
+    } else {
+      RTR_TRY(ensure_layers());
+      hipLaunchKernelGGL(k_pack_multi, dim3(2048), dim3(256), 0, stream, pts.as<float>(), n, k, rots.as<float>(),
+                         x0.as<uint16_t>());
+      enqueue_point_mlp_layers(C);
+      hipLaunchKernelGGL(k_concat_multi, dim3(B), dim3(2 * kC3), 0, stream, G.as<float>(), n, k, F.as<uint16_t>());
+    }
     gemm(stream, F.as<uint16_t>(), 2 * kC3, 0, wbp(L.W4), kH, 0, h1.p, kH, B, kH, 2 * kC3, wp(L.b4), 1, 1);
     gemm(stream, h1.as<uint16_t>(), kH, 0, wbp(L.W5), kOut, 0, O.p, kOut, B, kOut, kH, wp(L.b5), 0, 0);
-    hipLaunchKernelGGL(k_head, dim3((B + 63) / 64), dim3(64), 0, stream, O.as<float>(), B, pts.as<float>(),
-                       nullptr, pose.as<double>(), nullptr, nullptr);
+    hipLaunchKernelGGL(k_head, dim3((B + 63) / 64), dim3(64), 0, stream, O.as<float>(), B, nullptr, nullptr,
+                       pose.as<double>(), nullptr, nullptr);
     hipLaunchKernelGGL(k_score, dim3(B), dim3(256), 0, stream, pts.as<float>(), pose.as<double>(),
                        rots.as<float>(), n, k, tau2, score.as<double>());
+    return RTR_OK;
   }
 
   // gradients of the mean loss into g (FP32)
   void enqueue_backward() {
     const int B = n_pairs, C = 2 * B;
-    const size_t rows = (size_t)C * kP;
     float* gp = g.as<float>();
-    hipLaunchKernelGGL(k_zero, dim3(256), dim3(256), 0, stream, gp, L.total);
-    const unsigned cs_blocks = 64;
     // head layer 2: O = H1 W5 + b5
     hipLaunchKernelGGL(k_to_bf16, dim3(64), dim3(256), 0, stream, dO.as<float>(), (size_t)B * kOut,
                        dOb.as<uint16_t>());
     gemm(stream, h1.as<uint16_t>(), kH, 1, dOb.as<uint16_t>(), kOut, 0, gp + L.W5, kOut, kH, kOut, B, nullptr, 0, 0);
-    hipLaunchKernelGGL(k_colsum_f32, dim3(1, 1), dim3(64), 0, stream, dO.as<float>(), (size_t)B, kOut, gp + L.b5);
+    hipLaunchKernelGGL(k_colsum<float>, dim3(1), dim3(1024), 0, stream, dO.as<float>(), B, kOut, gp + L.b5);
     gemm(stream, dOb.as<uint16_t>(), kOut, 0, wbp(L.W5), kOut, 1, dH1.p, kH, B, kH, kOut, nullptr, 0, 0);
     hipLaunchKernelGGL(k_relu_back, dim3(64), dim3(256), 0, stream, dH1.as<float>(), h1.as<uint16_t>(),
                        (size_t)B * kH, dH1b.as<uint16_t>());
     // head layer 1: H1 = relu(F W4 + b4)
     gemm(stream, F.as<uint16_t>(), 2 * kC3, 1, dH1b.as<uint16_t>(), kH, 0, gp + L.W4, kH, 2 * kC3, kH, B, nullptr,
          0, 0);
-    hipLaunchKernelGGL(k_colsum, dim3(1, 1), dim3(kH), 0, stream, dH1b.as<uint16_t>(), (size_t)B, kH, gp + L.b4);
+    hipLaunchKernelGGL(k_colsum<uint16_t>, dim3(kH / 64), dim3(1024), 0, stream, dH1b.as<uint16_t>(), B, kH,
+                       gp + L.b4);
     gemm(stream, dH1b.as<uint16_t>(), kH, 0, wbp(L.W4), kH, 1, dF.p, 2 * kC3, B, 2 * kC3, kH, nullptr, 0, 0);
-    hipLaunchKernelGGL(k_split, dim3(B), dim3(2 * kC3), 0, stream, dF.as<float>(), B, dG.as<float>());
-    // max-pool + ReLU: dY3 nonzero at the argmax rows only
-    hipLaunchKernelGGL(k_pool_back, dim3(2048), dim3(256), 0, stream, dG.as<float>(), arg.as<int32_t>(),
-                       G.as<float>(), kC3, rows, dbf.as<uint16_t>());
-    const int ks = (int)std::min<size_t>(256, rows / 1024 + 1);
-    // layer 3: Y3 = relu(Y2 W3 + b3)
-    gemm(stream, y2.as<uint16_t>(), kC2, 1, dbf.as<uint16_t>(), kC3, 0, gp + L.W3, kC3, kC2, kC3, (int)rows, nullptr,
-         0, 0, ks);
-    hipLaunchKernelGGL(k_colsum, dim3(cs_blocks, 1), dim3(kC3), 0, stream, dbf.as<uint16_t>(), rows, kC3, gp + L.b3);
-    gemm(stream, dbf.as<uint16_t>(), kC3, 0, wbp(L.W3), kC3, 1, dtmp.p, kC2, (int)rows, kC2, kC3, nullptr, 0, 0);
-    hipLaunchKernelGGL(k_relu_back, dim3(1024), dim3(256), 0, stream, dtmp.as<float>(), y2.as<uint16_t>(),
-                       rows * kC2, dbf.as<uint16_t>());
-    // layer 2
-    gemm(stream, y1.as<uint16_t>(), kC1, 1, dbf.as<uint16_t>(), kC2, 0, gp + L.W2, kC2, kC1, kC2, (int)rows, nullptr,
-         0, 0, ks);
-    hipLaunchKernelGGL(k_colsum, dim3(cs_blocks, 1), dim3(kC2), 0, stream, dbf.as<uint16_t>(), rows, kC2, gp + L.b2);
-    gemm(stream, dbf.as<uint16_t>(), kC2, 0, wbp(L.W2), kC2, 1, dtmp.p, kC1, (int)rows, kC1, kC2, nullptr, 0, 0);
-    hipLaunchKernelGGL(k_relu_back, dim3(1024), dim3(256), 0, stream, dtmp.as<float>(), y1.as<uint16_t>(),
-                       rows * kC1, dbf.as<uint16_t>());
-    // layer 1
-    gemm(stream, x0.as<uint16_t>(), kC0, 1, dbf.as<uint16_t>(), kC1, 0, gp + L.W1, kC1, kC0, kC1, (int)rows, nullptr,
-         0, 0, ks);
-    hipLaunchKernelGGL(k_colsum, dim3(cs_blocks, 1), dim3(kC1), 0, stream, dbf.as<uint16_t>(), rows, kC1, gp + L.b1);
+    // point MLP (W1 .. b3 are the parameters' first kBackParams)
+    const int grid = C < fused_blocks ? C : fused_blocks;
+    hipLaunchKernelGGL(k_mlp_back, dim3(grid), dim3(kBackThreads), sizeof(BackShared), stream, pts.as<float>(), C,
+                       wb.as<uint16_t>(), w.as<float>(), L, dF.as<float>(), arg.as<int32_t>(), G.as<float>(),
+                       back.as<float>());
+    hipLaunchKernelGGL(k_sum_partials, dim3((unsigned)((kBackParams + 63) / 64)), dim3(256), 0, stream,
+                       back.as<float>(), grid, kBackParams, gp);
   }
 
   int upload_labels(const double* labels) {
@@ -1433,7 +1775,7 @@ int rtr_prop_propose(rtr_prop* h, double* poses) {
   }
   RTR_HIP(hipEventRecord(P.ev0, P.stream));
   P.enqueue_fps();
-  P.enqueue_forward(false, P.fused_off);
+  RTR_TRY(P.enqueue_forward(false));
   RTR_HIP(hipGetLastError());
   RTR_HIP(hipEventRecord(P.ev1, P.stream));
   std::vector<double> pose((size_t)P.n_pairs * 12);
@@ -1497,7 +1839,7 @@ int rtr_prop_propose_multi(rtr_prop* h, int k, const double* rots_in, float tau,
   RTR_HIP(hipMemcpyAsync(P.rots.p, rf, (size_t)k * 9 * 4, hipMemcpyHostToDevice, P.stream));
   RTR_HIP(hipEventRecord(P.ev0, P.stream));
   P.enqueue_fps();
-  P.enqueue_forward_multi(k, tau * tau);
+  RTR_TRY(P.enqueue_forward_multi(k, tau * tau));
   RTR_HIP(hipGetLastError());
   RTR_HIP(hipEventRecord(P.ev1, P.stream));
   // read back through pinned staging (poses, scores, centroids)
@@ -1578,7 +1920,7 @@ int rtr_prop_forward_backward(rtr_prop* h, int n_pairs, const float* xyz, const 
   if (!rc) rc = P.set_points(n_pairs, xyz);
   if (rc) return rc;
   if (labels) RTR_HIP(hipMemcpyAsync(P.lab.p, labels, (size_t)n_pairs * 12 * 8, hipMemcpyHostToDevice, P.stream));
-  P.enqueue_forward(labels != nullptr, labels != nullptr || P.fused_off);
+  RTR_TRY(P.enqueue_forward(labels != nullptr));
   if (labels && grad_out) P.enqueue_backward();
   RTR_HIP(hipGetLastError());
   if (O_out) RTR_HIP(hipMemcpyAsync(O_out, P.O.p, (size_t)n_pairs * kOut * 4, hipMemcpyDeviceToHost, P.stream));
@@ -1604,7 +1946,7 @@ int rtr_prop_train_step(rtr_prop* h, int n_pairs, const float* xyz, const double
   if (!rc) rc = P.set_points(n_pairs, xyz);
   if (rc) return rc;
   RTR_HIP(hipMemcpyAsync(P.lab.p, labels, (size_t)n_pairs * 12 * 8, hipMemcpyHostToDevice, P.stream));
-  P.enqueue_forward(true, true);
+  RTR_TRY(P.enqueue_forward(true));
   P.enqueue_backward();
   P.step += 1;
   const float b1 = 0.9f, b2 = 0.999f;

@@ -382,3 +382,45 @@ def test_hardware_bf16_conversion_matches_software_rounding():
     n = C.c_ulonglong(1)
     L.check(L.lib.rtr_bf16_conversion_check(0, C.byref(n)))
     assert n.value == 0
+
+
+def _cloud_points(kind, n, rng):
+    """n pairs of centred 1024-point clouds with the active rows a backward can meet."""
+    x = rng.normal(0, 0.4, (2 * n, learned.KP, 3))
+    if kind == "few_points":          # 5 distinct points: ties everywhere, one tile
+        x = x[:, rng.integers(0, 5, learned.KP)]
+    elif kind == "one_point":         # a single active row per cloud
+        x = np.repeat(x[:, :1], learned.KP, axis=1)
+    return x.astype(np.float32).reshape(-1, 3)
+
+
+@pytest.mark.parametrize("kind,n,bias3", [("spread", 1, 0.0), ("spread", 3, 0.0), ("few_points", 2, 0.0),
+                                          ("one_point", 2, 0.0), ("spread", 2, -1e3), ("spread", 2, -0.4),
+                                          ("spread", 129, 0.0)])
+def test_gradient_over_active_rows_matches_oracle(kind, n, bias3):
+    """The point MLP's backward runs over the argmax rows only: many of them
+    (several tiles and a remainder), few, one, none (a third-layer bias that
+    silences every channel, or some), and more clouds than workgroups."""
+    rng = np.random.default_rng(31 + n)
+    xyz = _cloud_points(kind, n, rng)
+    lab = _labels(rng, n)
+    w = learned.init_weights(5)
+    w[-9:] += rng.normal(0, 0.3, 9).astype(np.float32)
+    off = {}
+    o = 0
+    for name, shp in mlp._SHAPES:
+        off[name] = (o, o + int(np.prod(shp)))
+        o = off[name][1]
+    w[slice(*off["b3"])] += np.float32(bias3)
+    got = learned.Proposer(max_pairs=n, weights=w).forward_backward(xyz, lab)
+    ref = mlp.forward_backward(w, xyz, lab, emulate_bf16=True)
+    assert _rel(got["O"], ref["O"]) < 1e-3
+    # a BF16 rounding that falls the other way moves one stored value by 2^-8:
+    # the bound of the dense gradient's test
+    for name, (a, b) in off.items():
+        if np.linalg.norm(ref["grad"][a:b]) > 0:
+            assert _rel(got["grad"][a:b], ref["grad"][a:b]) < 2e-2, name
+        else:
+            assert not np.any(got["grad"][a:b]), name
+    assert _rel(got["grad"], ref["grad"]) < 1e-2
+
