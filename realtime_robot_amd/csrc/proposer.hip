@@ -76,7 +76,7 @@ struct ParamLayout {
 //   A(i,k) = ta ? A[k*lda + i] : A[i*lda + k]   (bf16)
 //   B(k,j) = tb ? B[j*ldb + k] : B[k*ldb + j]   (bf16)
 // Output FP32 (atomicAdd when split-K) or BF16.  64 x 64 tile per workgroup
-// (2 x 2 waves of 32 x 32 MFMA tiles), K staged through LDS 32 at a time.
+// (2 x 2 waves of 32 x 32 MFMA tiles), K staged through LDS 64 at a time.
 // ---------------------------------------------------------------------------
 struct GemmArgs {
   const uint16_t* A;
@@ -87,12 +87,37 @@ struct GemmArgs {
   int ta, tb, relu, out_bf16, atomic_out, k_split;
 };
 
-constexpr int kTM = 64, kTN = 64, kTK = 32;
+constexpr int kTM = 64, kTN = 64, kTK = 64;
+constexpr int kTPad = 8;  // row padding: 16-byte aligned rows
 
+// Eight elements i .. i + 7 of row j of a row-major matrix (rows x cols, row
+// stride ld), zero outside: one 16-byte load where all are inside and the
+// address allows it (vec), else element by element.
+__device__ __forceinline__ uint4 load8(const uint16_t* M, int ld, int rows, int cols, int j, int i, bool vec) {
+  union {
+    uint4 v;
+    uint16_t e[8];
+  } o;
+  o.v = make_uint4(0u, 0u, 0u, 0u);
+  if (j >= rows || i >= cols) return o.v;
+  const uint16_t* q = M + (size_t)j * ld + i;
+  if (vec && i + 8 <= cols) return *reinterpret_cast<const uint4*>(q);
+#pragma unroll
+  for (int u = 0; u < 8; ++u)
+    if (i + u < cols) o.e[u] = q[u];
+  return o.v;
+}
+
+// The K steps of a tile: both operands go to LDS as [row or column][k], so
+// that a lane's four consecutive k are one 8-byte read.  The next step's
+// 16-byte loads are in flight while this one multiplies.  The products here
+// are small (a head of 256-2048 rows: 16-128 workgroups), so what bounds them
+// is the latency of K / 64 dependent steps: the six products of a 256-pair
+// gradient took 32 us each on average with element loads, two barriers per 32
+// k and nothing in flight, 17 us now.
 __global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g) {
-  // rows padded by 4 elements (8 B): 8-byte aligned bf16x4 operand reads
-  __shared__ __align__(16) uint16_t sA[kTM][kTK + 4];
-  __shared__ __align__(16) uint16_t sBt[kTN][kTK + 4];
+  __shared__ __align__(16) uint16_t sA[kTM][kTK + kTPad];
+  __shared__ __align__(16) uint16_t sBt[kTN][kTK + kTPad];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   const int wm = w >> 1, wn = w & 1;
   const int m0 = blockIdx.x * kTM, n0 = blockIdx.y * kTN;
@@ -100,42 +125,41 @@ __global__ __launch_bounds__(256) void k_gemm_bf16(GemmArgs g) {
   const int kchunk = ((g.K + g.k_split - 1) / g.k_split + kTK - 1) / kTK * kTK;
   const int kb = blockIdx.z * kchunk;
   const int ke = min(g.K, kb + kchunk);
+  const bool va = (g.lda & 7) == 0 && (reinterpret_cast<uintptr_t>(g.A) & 15) == 0;
+  const bool vb = (g.ldb & 7) == 0 && (reinterpret_cast<uintptr_t>(g.B) & 15) == 0;
+  // two 8-element pieces of each operand per thread: along k where the
+  // operand's rows run along k, along its M (N) dimension else
+  const int pj = tid >> 3, pi = (tid & 7) * 8;
+  uint4 ra[2], rb[2];
+  auto load = [&](int k0) {
+#pragma unroll
+    for (int u = 0; u < 2; ++u) {
+      const int j = pj + 32 * u;
+      ra[u] = g.ta ? load8(g.A, g.lda, ke, g.M, k0 + j, m0 + pi, va) : load8(g.A, g.lda, g.M, ke, m0 + j, k0 + pi, va);
+      rb[u] = g.tb ? load8(g.B, g.ldb, g.N, ke, n0 + j, k0 + pi, vb) : load8(g.B, g.ldb, ke, g.N, k0 + j, n0 + pi, vb);
+    }
+  };
+  auto store = [&](uint16_t(*d)[kTK + kTPad], const uint4& v, int j, bool along_k) {
+    if (along_k) {
+      *reinterpret_cast<uint4*>(&d[j][pi]) = v;
+    } else {
+      const uint16_t* e = reinterpret_cast<const uint16_t*>(&v);
+#pragma unroll
+      for (int u = 0; u < 8; ++u) d[pi + u][j] = e[u];
+    }
+  };
   f32x16 acc;
 #pragma unroll
   for (int j = 0; j < 16; ++j) acc[j] = 0.f;
+  if (kb < ke) load(kb);
   for (int k0 = kb; k0 < ke; k0 += kTK) {
-    // stage A (64 x 32) and B (32 x 64, stored transposed): 2048 elements
-    // each, 8 per thread; consecutive threads walk the operand's contiguous
-    // dimension
 #pragma unroll
-    for (int e = 0; e < 8; ++e) {
-      const int idx = tid + e * 256;
-      int r, c;  // A tile row r (M), column c (K)
-      if (g.ta) {
-        r = idx % kTM;
-        c = idx / kTM;
-      } else {
-        r = idx / kTK;
-        c = idx % kTK;
-      }
-      const int gi = m0 + r, gk = k0 + c;
-      uint16_t v = 0;
-      if (gi < g.M && gk < ke) v = g.ta ? g.A[(size_t)gk * g.lda + gi] : g.A[(size_t)gi * g.lda + gk];
-      sA[r][c] = v;
-      int rk, cn;  // B tile row rk (K), column cn (N)
-      if (g.tb) {
-        rk = idx % kTK;
-        cn = idx / kTK;
-      } else {
-        rk = idx / kTN;
-        cn = idx % kTN;
-      }
-      const int gk2 = k0 + rk, gj = n0 + cn;
-      uint16_t u = 0;
-      if (gk2 < ke && gj < g.N) u = g.tb ? g.B[(size_t)gj * g.ldb + gk2] : g.B[(size_t)gk2 * g.ldb + gj];
-      sBt[cn][rk] = u;
+    for (int u = 0; u < 2; ++u) {
+      store(sA, ra[u], pj + 32 * u, !g.ta);
+      store(sBt, rb[u], pj + 32 * u, g.tb);
     }
     __syncthreads();
+    if (k0 + kTK < ke) load(k0 + kTK);
 #pragma unroll
     for (int kk = 0; kk < kTK; kk += 8) {
       const int kq = kk + (lane >> 5) * 4;

@@ -424,3 +424,11 @@ def test_gradient_over_active_rows_matches_oracle(kind, n, bias3):
             assert not np.any(got["grad"][a:b]), name
     assert _rel(got["grad"], ref["grad"]) < 1e-2
 
+
+@pytest.mark.parametrize("M,N,K,ta,tb,ks", [
+    (64, 64, 64, 0, 0, 1), (65, 72, 64, 0, 0, 1), (8, 264, 72, 0, 1, 1), (72, 8, 136, 1, 0, 1), (136, 56, 63, 1, 1, 1),
+    (1, 1, 1, 0, 0, 1), (63, 65, 200, 0, 1, 2), (128, 128, 513, 1, 1, 5), (256, 9, 256, 0, 0, 1), (40, 16, 8, 0, 0, 4)])
+def test_gemm_bf16_wide_loads(M, N, K, ta, tb, ks):
+    """Edges of the 64 x 64 x 64 tiles, with leading dimensions that allow the
+    16-byte loads and ones that do not, and K splits with empty parts."""
+    test_gemm_bf16_matches_numpy(M, N, K, ta, tb, ks)
