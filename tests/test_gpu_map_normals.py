@@ -245,3 +245,42 @@ def test_streaming_reconstruction_tracks_the_camera():
           f"states {states}")
     assert ate < 0.02 and rot < 1.0
     assert all(1 <= st <= 4 for st in states) and rec.map.dropped() == 0
+
+
+@pytest.mark.parametrize("shape,n", [("room", 40000), ("room", 3), ("one", 500), ("line", 3000), ("negative", 5000),
+                                     ("sparse", 2000), ("two_far", 2)])
+def test_map_readout_order_and_reuse(shape, n):
+    """Keys in ascending order with their counts and centroids, through the
+    bit map of the key box (room-sized boxes, single voxels, lines) and
+    through the host's sort (boxes too sparse for it), again after a clear of
+    few voxels and of many, and the same order from the downsample."""
+    rng = np.random.default_rng(n)
+    p = rng.uniform(0, 1, (n, 3)) * {"room": [5, 5, 2.5], "one": [0.009, 0.009, 0.009], "line": [9, 0.01, 0.01],
+                                     "negative": [2, 3, 1], "sparse": [900, 900, 900], "two_far": [9000, 9000, 9000]}[shape]
+    if shape == "negative":
+        p -= [1.5, 3.0, 0.25]
+    p = p.astype(np.float32)
+    h = np.float32(0.02) if shape != "one" else np.float32(0.01)
+    inv = np.float32(1.0 / float(h))
+    k = np.floor(p * inv).astype(np.int64) + (1 << 20)
+    key = k[:, 0] | (k[:, 1] << 21) | (k[:, 2] << 42)
+    keys, where, counts = np.unique(key, return_inverse=True, return_counts=True)
+    mean = np.stack([np.bincount(where, p[:, a].astype(np.float64)) / counts for a in range(3)], 1)
+    # the float result, and offsets of up to a voxel summed in floats
+    tol = 1.2e-7 * np.abs(mean) + 2e-6
+    m = R.VoxelMap(float(h), capacity=max(n, 64))   # the larger clouds fill more than an eighth of the slots
+    for rep in range(3):
+        m.integrate(p)
+        gk, gx, gc = m.extract()
+        assert np.array_equal(gk, keys) and np.array_equal(gc, counts)
+        assert np.all(np.abs(gx - mean) <= tol)
+        m.clear()
+        assert m.size() == 0 and len(m.extract()[0]) == 0
+        m.integrate(p[:2])
+        assert m.size() == len(np.unique(key[:2]))
+        m.clear()
+    m.integrate(p)
+    _, sums, _ = m.extract(centroids=False)
+    assert np.allclose(sums, mean * counts[:, None], rtol=2e-7, atol=2e-6 * counts.max())
+    d = R.voxel_downsample(p, float(h))
+    assert d.shape == mean.shape and np.all(np.abs(d - mean) <= tol)
