@@ -13,6 +13,7 @@
 // to floor((p - origin) * (1 / resolution)) in FP32.
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cstring>
 #include <mutex>
 #include <vector>
@@ -49,83 +50,102 @@ __global__ void k_tdf_mark_points(const float* xyz, size_t n, float ox, float oy
   }
 }
 
-// One pass along axis A (0 = x, 1 = y, 2 = z): out(a) = min_t (a - t)^2 + in(t)
-// over the line through the voxel; the line is staged in LDS one 1024-value
-// tile at a time.  The last pass applies the cap.
+// One pass along axis A (0 = x, 1 = y, 2 = z): out(a) = min(cap, min_t
+// (a - t)^2 + in(t)) over the line through the voxel, one voxel per lane.  The
+// offsets go outward and stop at the first r with r^2 >= the best so far: no
+// farther term can be smaller (its rounded sum is at least r^2), so the result
+// is that of the whole line, bit for bit.  Capping every pass, not the last
+// alone, changes nothing either (a term with in >= cap is >= cap) and bounds
+// the offsets by sqrt(cap) where a line holds nothing.  Lanes run along x, so
+// every load of the three passes is one contiguous segment per wave; four
+// offsets to each side are in flight at once.
+//
+// Staging whole lines in LDS and taking all len terms (len^2 per line) was
+// VALU-bound: 405, 411 and 231 us for 250 x 250 x 125 at cap 900; 95, 94 and 124 now,
+// bound by the latency of the loads (the field is 31 MB: L2 and MALL).
 template <int A>
-__global__ __launch_bounds__(256) void k_tdf_pass(const float* in, float* out, int dx, int dy, int dz, float cap) {
-  __shared__ float line[1024];
-  const int len = A == 0 ? dx : (A == 1 ? dy : dz);
-  // lines are enumerated by the two other coordinates
-  const size_t n_lines = (size_t)dx * dy * dz / (size_t)len;
-  for (size_t li = blockIdx.x; li < n_lines; li += gridDim.x) {
-    size_t base, stride;
-    if (A == 0) {
-      base = li * dx;
-      stride = 1;
-    } else if (A == 1) {
-      const size_t x = li % dx, z = li / dx;
-      base = x + (size_t)dx * dy * z;
-      stride = dx;
-    } else {
-      base = li;
-      stride = (size_t)dx * dy;
-    }
-    for (int a0 = 0; a0 < len; a0 += 256) {
-      const int a = a0 + threadIdx.x;
-      float best = kTdfInf;
-      for (int t0 = 0; t0 < len; t0 += 1024) {
-        const int tn = min(1024, len - t0);
-        __syncthreads();
-        for (int t = threadIdx.x; t < tn; t += 256) line[t] = in[base + (size_t)(t0 + t) * stride];
-        __syncthreads();
-        if (a < len) {
-          for (int t = 0; t < tn; ++t) {
-            const float d = (float)(a - (t0 + t));
-            best = fminf(best, d * d + line[t]);
-          }
-        }
+__global__ __launch_bounds__(256) void k_tdf_pass(const float* in, float* out, uint32_t n, int dx, int dy, int dz,
+                                                  float cap) {
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
+    const uint32_t q = i / (uint32_t)dx;
+    const int pos = A == 0 ? (int)(i - q * (uint32_t)dx) : (A == 1 ? (int)(q % (uint32_t)dy) : (int)(q / (uint32_t)dy));
+    const int len = A == 0 ? dx : (A == 1 ? dy : dz);
+    const ptrdiff_t stride = A == 0 ? 1 : (A == 1 ? dx : (ptrdiff_t)dx * dy);
+    const float* p = in + i;
+    const int lo = pos, hi = len - 1 - pos, far = lo > hi ? lo : hi;  // offsets inside the line
+    float best = fminf(*p, cap);
+    for (int r = 1; r <= far && (float)r * (float)r < best; r += 4) {
+      float a[4], b[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        a[u] = p[-(ptrdiff_t)min(r + u, lo) * stride];
+        b[u] = p[(ptrdiff_t)min(r + u, hi) * stride];
       }
-      if (a < len) out[base + (size_t)a * stride] = cap > 0.f ? fminf(best, cap) : best;
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        // (an offset past the line's end repeats the end voxel's value at a
+        // larger distance than its own: never below the term it stands for)
+        const float d = (float)(r + u) * (float)(r + u);
+        best = fminf(best, fminf(d + a[u], d + b[u]));
+      }
     }
+    out[i] = best;
   }
+}
+
+// The three passes over n = dx dy dz <= 2^31 voxels, from a through b back to
+// a, and into out.
+static void tdf_passes(float* a, float* b, float* out, const int dims[3], float cap, hipStream_t s) {
+  const uint32_t n = (uint32_t)((size_t)dims[0] * dims[1] * dims[2]);
+  const dim3 g(std::min((n + 255u) / 256u, 1u << 20)), t(256);
+  hipLaunchKernelGGL(k_tdf_pass<0>, g, t, 0, s, a, b, n, dims[0], dims[1], dims[2], cap);
+  hipLaunchKernelGGL(k_tdf_pass<1>, g, t, 0, s, b, a, n, dims[0], dims[1], dims[2], cap);
+  hipLaunchKernelGGL(k_tdf_pass<2>, g, t, 0, s, a, out, n, dims[0], dims[1], dims[2], cap);
+}
+
+// Fills, marks, transforms and reads back; mem holds two fields and the input.
+static int tdf_enqueue(float* mem, const int dims[3], float trunc2, float* out, const int32_t* occ, size_t n_occ,
+                       const float* xyz, size_t n_pts, size_t stride, const float origin[3], float res) {
+  const int dx = dims[0], dy = dims[1], dz = dims[2];
+  const size_t n = (size_t)dx * dy * dz;
+  float* const a = mem;
+  float* const b = mem + n;
+  float* const src = mem + 2 * n;
+  hipStream_t s = nullptr;
+  hipLaunchKernelGGL(k_tdf_fill, dim3((unsigned)std::min<size_t>(1024, (n + 255) / 256)), dim3(256), 0, s, a, n);
+  if (occ && n_occ) {
+    RTR_HIP(hipMemcpy(src, occ, n_occ * 12, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_tdf_mark, dim3(256), dim3(256), 0, s, reinterpret_cast<int32_t*>(src), n_occ, dx, dy, dz, a);
+  } else if (xyz && n_pts) {
+    std::vector<float> packed;
+    const float* from = xyz;
+    if (stride != 12) {
+      packed.resize(3 * n_pts);
+      const char* base = reinterpret_cast<const char*>(xyz);
+      for (size_t i = 0; i < n_pts; ++i) memcpy(&packed[3 * i], base + i * stride, 12);
+      from = packed.data();
+    }
+    RTR_HIP(hipMemcpy(src, from, n_pts * 12, hipMemcpyHostToDevice));
+    hipLaunchKernelGGL(k_tdf_mark_points, dim3(256), dim3(256), 0, s, src, n_pts, origin[0], origin[1], origin[2],
+                       1.0f / res, dx, dy, dz, a);
+  }
+  tdf_passes(a, b, b, dims, trunc2, s);
+  RTR_HIP(hipGetLastError());
+  RTR_HIP(hipMemcpy(out, b, n * 4, hipMemcpyDeviceToHost));
+  return RTR_OK;
 }
 
 static int tdf_run(int device, const int dims[3], float trunc2, float* out, const int32_t* occ, size_t n_occ,
                    const float* xyz, size_t n_pts, size_t stride, const float origin[3], float res) {
   RTR_HIP(hipSetDevice(device));
-  const int dx = dims[0], dy = dims[1], dz = dims[2];
-  const size_t n = (size_t)dx * dy * dz;
-  DevBuf a, b, src;
-  int rc = a.ensure(n * 4);
-  if (!rc) rc = b.ensure(n * 4);
+  const size_t n = (size_t)dims[0] * dims[1] * dims[2];
+  // one allocation: the two fields, then the input
   const size_t src_bytes = occ ? n_occ * 12 : n_pts * 12;
-  if (!rc && src_bytes) rc = src.ensure(src_bytes);
-  if (rc) return rc;
-  hipStream_t s = nullptr;
-  hipLaunchKernelGGL(k_tdf_fill, dim3(1024), dim3(256), 0, s, a.as<float>(), n);
-  if (occ && n_occ) {
-    RTR_HIP(hipMemcpy(src.p, occ, n_occ * 12, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_tdf_mark, dim3(256), dim3(256), 0, s, src.as<int32_t>(), n_occ, dx, dy, dz, a.as<float>());
-  } else if (xyz && n_pts) {
-    std::vector<float> packed(3 * n_pts);
-    const char* base = reinterpret_cast<const char*>(xyz);
-    for (size_t i = 0; i < n_pts; ++i) memcpy(&packed[3 * i], base + i * stride, 12);
-    RTR_HIP(hipMemcpy(src.p, packed.data(), n_pts * 12, hipMemcpyHostToDevice));
-    hipLaunchKernelGGL(k_tdf_mark_points, dim3(256), dim3(256), 0, s, src.as<float>(), n_pts, origin[0], origin[1],
-                       origin[2], 1.0f / res, dx, dy, dz, a.as<float>());
-  }
-  const unsigned blocks = 2048;
-  hipLaunchKernelGGL(k_tdf_pass<0>, dim3(blocks), dim3(256), 0, s, a.as<float>(), b.as<float>(), dx, dy, dz, 0.f);
-  hipLaunchKernelGGL(k_tdf_pass<1>, dim3(blocks), dim3(256), 0, s, b.as<float>(), a.as<float>(), dx, dy, dz, 0.f);
-  hipLaunchKernelGGL(k_tdf_pass<2>, dim3(blocks), dim3(256), 0, s, a.as<float>(), b.as<float>(), dx, dy, dz,
-                     trunc2);
-  RTR_HIP(hipGetLastError());
-  RTR_HIP(hipMemcpy(out, b.p, n * 4, hipMemcpyDeviceToHost));
-  a.release();
-  b.release();
-  src.release();
-  return RTR_OK;
+  DevBuf mem;
+  RTR_TRY(mem.ensure(2 * n * 4 + src_bytes));
+  const int rc = tdf_enqueue(mem.as<float>(), dims, trunc2, out, occ, n_occ, xyz, n_pts, stride, origin, res);
+  mem.release();
+  return rc;
 }
 
 // ---------------------------------------------------------------------------
@@ -212,12 +232,11 @@ int rtr_tdf_noalloc(int device, const int32_t* occ_dev, size_t n_occ, const int 
   const int dx = dims[0], dy = dims[1], dz = dims[2];
   // every scratch voxel is written by the fill before it is read: nothing
   // left by an earlier call on this device is used
+  // (the passes go from the caller's field to the scratch and back, so that
+  // the last one reads the scratch and writes the caller's)
   hipLaunchKernelGGL(k_tdf_fill, dim3(1024), dim3(256), 0, s, g, n);
   if (n_occ) hipLaunchKernelGGL(k_tdf_mark, dim3(256), dim3(256), 0, s, occ_dev, n_occ, dx, dy, dz, g);
-  const unsigned blocks = 2048;
-  hipLaunchKernelGGL(k_tdf_pass<0>, dim3(blocks), dim3(256), 0, s, g, out_dev, dx, dy, dz, 0.f);
-  hipLaunchKernelGGL(k_tdf_pass<1>, dim3(blocks), dim3(256), 0, s, out_dev, g, dx, dy, dz, 0.f);
-  hipLaunchKernelGGL(k_tdf_pass<2>, dim3(blocks), dim3(256), 0, s, g, out_dev, dx, dy, dz, trunc2);
+  tdf_passes(g, out_dev, out_dev, dims, trunc2, s);
   RTR_HIP(hipGetLastError());
   return RTR_OK;
 }

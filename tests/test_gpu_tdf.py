@@ -33,3 +33,17 @@ def test_tdf_of_key_point_box_like_the_reference():
     occ = np.unique(f[inside].astype(np.int32), axis=0)
     ref = oracle.tdf(occ, (30, 30, 30), 900.0)
     assert len(occ) > 50 and np.array_equal(got, ref)
+
+
+@pytest.mark.parametrize("dims", [(1, 1, 1), (2, 1, 3), (5, 4, 1), (6, 9, 13), (700, 1, 2), (1, 66, 1), (3, 2, 259)])
+@pytest.mark.parametrize("cap", [0.25, 1.0, 30.5, 900.0, 1.0e9])
+def test_outward_passes_match_brute_force(dims, cap):
+    """Lines shorter than, as long as and just beyond the four offsets taken
+    at a time, caps below one voxel, between whole numbers and out of reach,
+    one voxel occupied, all of one face, and none."""
+    rng = np.random.default_rng(sum(dims))
+    d = np.array(dims)
+    one = (rng.random((1, 3)) * d).astype(np.int32)
+    face = np.stack([np.zeros(8, np.int32), *(rng.integers(0, d[a], 8) for a in (1, 2))], 1).astype(np.int32)
+    for occ in (one, face, np.zeros((0, 3), np.int32)):
+        assert np.array_equal(R.tdf(occ, dims, cap), oracle.tdf(occ, dims, cap))
