@@ -118,6 +118,7 @@ int rtr_icp_create(rtr_icp** out, int device) {
   // sums.
   h->eng.tune().item_pts = 256;
   h->eng.tune().blocks_per_cu = 1;
+  h->eng.tune().single = true;
   *out = h;
   return RTR_OK;
   RTR_GUARD_END

@@ -359,7 +359,7 @@ int Engine::layout_problems() {
   // longest-first on the least-loaded XCD.
   items_.clear();
   pt_total_ = 0;
-  const uint32_t ip = (uint32_t)tune_.item_pts;
+  const uint32_t ip = item_points();
   std::vector<uint64_t> tload(tgts_.size(), 0);
   for (const Problem& pr : probs_) tload[pr.tgt] += (srcs_[pr.src].n + ip - 1) / ip;
   std::vector<int> order(tgts_.size());
@@ -486,7 +486,8 @@ DevEngine Engine::dev_view() const {
   e.nn_seed = (pt_total_ > 0 && pt_total_ <= 0xffffffffull) ? nn_seed_.as<uint32_t>() : nullptr;
   e.items = items_buf_.as<uint2>();
   e.n_items = (int)items_.size();
-  e.item_pts = tune_.item_pts;
+  e.item_pts = (int)item_points();
+  e.one = one_problem() ? 1 : 0;
   e.use_tile = tune_.use_tile;
   e.variant = variant();
   e.retire_from = tune_.retire > 0.f ? cu_count_ : 0x7fffffff;
@@ -529,7 +530,26 @@ DevEngine Engine::dev_view() const {
   return e;
 }
 
+// The one-registration kernel serves engines set up for single registrations
+// (TuneParams::single) while 256 queries' worth of workgroups on every CU reach
+// the whole source in a few rounds; beyond a million points the work, not the
+// chain of iterations, is what a launch waits for.
+bool Engine::one_problem() const {
+  return tune_.single && probs_.size() == 1 && srcs_[probs_[0].src].n <= (1u << 20);
+}
+
+// Points per work item: as tuned, or for one problem 64 (one query per four
+// lanes of a workgroup) as long as the items fit the workgroups that can be
+// resident, else the next multiple of 64 that does.
+uint32_t Engine::item_points() const {
+  if (!one_problem()) return (uint32_t)tune_.item_pts;
+  const uint32_t n = srcs_[probs_[0].src].n;
+  const uint32_t most = std::min<uint32_t>((uint32_t)(cu_count_ * std::min(2, icp_one_blocks_per_cu(prm_.mode))), kOneItems);
+  return 64u * std::max(1u, (n + 64u * most - 1u) / (64u * most));
+}
+
 int Engine::grid_blocks() const {
+  if (one_problem()) return std::max(1, (int)items_.size());
   int bpc = icp_blocks_per_cu(prm_.mode, tune_.use_tile, variant());
   if (tune_.blocks_per_cu > 0 && tune_.blocks_per_cu < bpc) bpc = tune_.blocks_per_cu;
   long long b = (long long)cu_count_ * bpc;

@@ -45,6 +45,7 @@ struct TuneParams {
   int blocks_per_cu = 0;          // persistent workgroups per CU (0 = occupancy limit)
   int use_tile = 0;               // LDS candidate tiles on/off
   float retire = 0.f;             // surplus workgroups leave below this fraction of unfinished problems
+  bool single = false;            // one registration per launch: a problem set of one runs k_icp_one
   int fine_from = 0;              // passes from this one on run 256-point work items (0: never)
 };
 
@@ -117,6 +118,10 @@ class Engine {
   int layout_targets();
   int layout_problems();
   int grid_blocks() const;
+  // one problem on the one-registration kernel: its items fit the kernel's
+  // list, and their size
+  bool one_problem() const;
+  uint32_t item_points() const;
 
   int device_;
   hipStream_t stream_ = nullptr;

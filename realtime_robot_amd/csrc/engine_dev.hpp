@@ -55,6 +55,7 @@ struct DevEngine {
   const uint2* items;        // (problem, first sorted source point)
   int n_items;
   int item_pts;              // points per item
+  int one;                   // one problem, searched by k_icp_one
   int use_tile;              // stage candidate tiles in LDS (else global gathers only)
   int variant;               // search kernel (point-to-point): 0 4-deep gathers at 3 waves per SIMD, 1 8-deep
                              // at 2, 2 4-deep at 4 (point-to-plane: always 8-deep at 2)
@@ -84,6 +85,8 @@ void launch_target_grid(const DevEngine& e, int max_tgt_pts, int max_cells, hipS
 void launch_source_sort(const DevEngine& e, int max_src_pts, uint32_t src_total, hipStream_t s);
 void launch_icp(const DevEngine& e, int grid_blocks, hipStream_t s);
 int icp_blocks_per_cu(int mode, int use_tile, int variant);
+int icp_one_blocks_per_cu(int mode);
+constexpr uint32_t kOneItems = 1024;  // most work items of a one-problem launch
 // correspondences / fitness / transformed output for problem set; T per
 // problem from `T` (n_prob*16 column-major, device) or from the state when null.
 void launch_correspondences(const DevEngine& e, int prob, const double* T, float r2f, int32_t* idx,

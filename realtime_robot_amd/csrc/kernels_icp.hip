@@ -51,6 +51,12 @@ constexpr int kMaxSpins = 1 << 22;
 __device__ __forceinline__ uint32_t load_relaxed(const uint32_t* p) {
   return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
 }
+__device__ __forceinline__ double load_relaxed(const double* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
+__device__ __forceinline__ int load_relaxed(const int* p) {
+  return __hip_atomic_load(p, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+}
 __device__ __forceinline__ void acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 __device__ __forceinline__ void store_release(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
@@ -353,6 +359,7 @@ template <int MODE, int NS, class TileT>
 __device__ void solve_problem(const DevEngine& e, uint32_t p, const Problem& pr,
                               const TargetDesc& td, int pass, IcpShared<NS, TileT>& sh) {
   const int tid = threadIdx.x;
+  constexpr uint32_t kGroups = kBlock / NSUM_MAX;
   const int v = tid % NSUM_MAX, grp = tid / NSUM_MAX;
   // the pose and the acceleration state are staged in LDS by the whole block
   // (one load per lane), so the single-thread FP64 work below reads no
@@ -364,9 +371,17 @@ __device__ void solve_problem(const DevEngine& e, uint32_t p, const Problem& pr,
   const bool fine = fine_pass(e, pass);
   const uint32_t i0 = first_item_of(pr, fine), ni = items_of(pr, fine);
   if (v < NS) {
-    for (uint32_t i = grp; i < ni; i += kBlock / NSUM_MAX) {
-      acc += e.partials[(size_t)(i0 + i) * NSUM_MAX + v];
+    // (added in item order; four loads in flight)
+    const double* q = e.partials + (size_t)i0 * NSUM_MAX + v;
+    uint32_t i = grp;
+    for (; i + 3 * kGroups < ni; i += 4 * kGroups) {
+      double t[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) t[u] = q[(size_t)(i + u * kGroups) * NSUM_MAX];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) acc += t[u];
     }
+    for (; i < ni; i += kGroups) acc += q[(size_t)i * NSUM_MAX];
   }
   sh.dred[grp][v] = acc;
   __syncthreads();
@@ -922,6 +937,266 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
   if (tid == 0) atomicAdd(e.queries_searched, (unsigned long long)sh.n_search);
 }
 
+// ---------------------------------------------------------------------------
+// One registration
+//
+// A launch of one problem is a chain of iterations, each as long as its
+// slowest item, the sums, the solve and the hand-over; throughput does not
+// matter.  So four lanes search one query: each takes every fourth row of the
+// ball, the four rows' points are then searched as one list, lane by lane, and
+// a workgroup holds 64 queries at a time.  Items are claimed in the first
+// iteration only and kept: a workgroup that starts late, or not until this
+// launch ends, leaves its share to those that run, so nothing waits for a
+// workgroup that is not resident; from then on there is no queue to ask.  While
+// it waits for the next transform a workgroup loads its queries, their seeds
+// and the seeds' points.  The transform is read with agent-scope loads and no
+// acquire: nothing else written during the launch is read by the search (its
+// seeds are the workgroup's own), so the target's cells stay in the L1 from
+// iteration to iteration.  A whole call on 2k x 10k points 1.70 -> 0.92 ms and
+// on 10k x 20k 2.23 -> 1.22 ms (38 -> 18 us an iteration, of which the sums and
+// the solve take 6); 30k x 366k points point-to-plane: the launch 1.0 -> 0.7 ms.
+// ---------------------------------------------------------------------------
+constexpr int kOneQueries = kBlock / 4;  // queries a workgroup searches at a time
+
+template <int I>
+__device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
+  return (uint32_t)dpp_i32<I * 0x55>((int)v);
+}
+
+// The quad's smallest key, and where it lies, in all four lanes.
+__device__ __forceinline__ void quad_min(uint64_t& key, uint32_t& where) {
+  uint64_t o = dpp_u64<kDppQuadXor1>(key);
+  uint32_t ow = (uint32_t)dpp_i32<kDppQuadXor1>((int)where);
+  where = o < key ? ow : where;
+  key = o < key ? o : key;
+  o = dpp_u64<kDppQuadXor2>(key);
+  ow = (uint32_t)dpp_i32<kDppQuadXor2>((int)where);
+  where = o < key ? ow : where;
+  key = o < key ? o : key;
+}
+
+// Four lanes search one query from its seed: key (and where, its slot) hold the
+// seed's on entry, equal in the four lanes, and the nearest point's on return.
+// Every cell that can hold a point within min(seed, r2f) is in the rows
+// [y0, y1] x [z0, z1]; each row is cut as in walk_ball, with the bound of the
+// rows before it.  All four lanes are active or none.
+__device__ __forceinline__ void search_quad(const GridView& g, float qx, float qy, float qz, float r2f, int sub,
+                                            uint64_t& key, uint32_t& where) {
+  float B = fminf(key_d2(key), r2f) * 1.000004f;
+  const float w = sqrt_approx(B) * 1.00001f + 2.0f * g.margin;
+  auto lo_of = [&](float q, float o) { return (int)fminf(fmaxf(((q - w) - o) * g.inv_h, 0.f), 1.0e9f); };
+  auto hi_of = [&](float q, float o, int n) {
+    return min((int)floorf(fminf(fmaxf(((q + w) - o) * g.inv_h, -1.f), 1.0e9f)), n - 1);
+  };
+  const int y0 = lo_of(qy, g.oy), ny = hi_of(qy, g.oy, g.dy) - y0 + 1;
+  const int z0 = lo_of(qz, g.oz), nz = hi_of(qz, g.oz, g.dz) - z0 + 1;
+  if (ny <= 0 || nz <= 0) return;
+  const int nrows = ny * nz;
+  const float inv_ny = 1.0f / (float)ny;
+  for (int r0 = 0; r0 < nrows; r0 += 4) {
+    const int r = r0 + sub;
+    // r / ny: exact, the callers keep nrows below 2^20 (the quotient's error
+    // stays far below the half that separates it from a whole number)
+    const int dz = (int)(((float)r + 0.5f) * inv_ny);
+    const int y = y0 + (r - dz * ny), z = z0 + dz;
+    const float gy = slab_gap(qy, g.oy, g.h, g.margin, y, y), gz = slab_gap(qz, g.oz, g.h, g.margin, z, z);
+    const float rem = B - (gy * gy + gz * gz);
+    uint32_t b = 0u, n = 0u;
+    if (r < nrows && rem >= 0.f) {
+      const float wx = sqrt_approx(rem) * 1.00001f + 2.0f * g.margin;
+      const int xa = (int)fminf(fmaxf(((qx - wx) - g.ox) * g.inv_h, 0.f), 1.0e9f);
+      const int xb = min((int)floorf(fminf(fmaxf(((qx + wx) - g.ox) * g.inv_h, -1.f), 1.0e9f)), g.dx - 1);
+      if (xa <= xb) {
+        const uint32_t row = ((uint32_t)z * g.dy + y) * g.dx;
+        b = g.cell_start[row + (uint32_t)xa];
+        n = g.cell_start[row + (uint32_t)xb + 1u] - b;
+      }
+    }
+    // the four rows' points as one list: point t is pts[t + base of its row]
+    const uint32_t n1 = quad_bcast<0>(n), n2 = n1 + quad_bcast<1>(n), n3 = n2 + quad_bcast<2>(n);
+    const uint32_t total = n3 + quad_bcast<3>(n);
+    const uint32_t b0 = quad_bcast<0>(b), b1 = quad_bcast<1>(b) - n1, b2 = quad_bcast<2>(b) - n2,
+                   b3 = quad_bcast<3>(b) - n3;
+    if (total == 0u) continue;
+    for (uint32_t t0 = 0; t0 < total; t0 += 16) {
+      float4 c[4];
+      uint32_t at[4];
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint32_t t = min(t0 + 4 * u + sub, total - 1u);  // past the end: the last point again
+        at[u] = t + (t < n1 ? b0 : (t < n2 ? b1 : (t < n3 ? b2 : b3)));
+        c[u] = g.pts[at[u]];
+      }
+#pragma unroll
+      for (int u = 0; u < 4; ++u) {
+        const uint64_t k = nn_key(d2_f32(qx, qy, qz, c[u].x, c[u].y, c[u].z), __float_as_int(c[u].w));
+        if (k < key) {
+          key = k;
+          where = at[u];
+        }
+      }
+    }
+    quad_min(key, where);
+    B = fminf(key_d2(key), r2f) * 1.000004f;
+  }
+}
+
+template <int MODE>
+__global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
+  constexpr int NS = MODE == RTR_MODE_POINT_TO_POINT ? SUM_P2P_COUNT : SUM_P2L_COUNT;
+  __shared__ IcpShared<NS, WaveTileNone> sh;
+  __shared__ uint16_t s_item[kOneItems];  // the items this workgroup keeps
+  const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, sub = tid & 3;
+  const Problem pr = scalar_copy(e.probs[0]);
+  const SourceDesc sd = scalar_copy(e.srcs[pr.src]);
+  const TargetDesc td = scalar_copy(e.tgts[pr.tgt]);
+  const GridView g = grid_of(e, td);
+  const float r2f = e.prm.r2f;
+  const double ax = (double)td.anchor[0], ay = (double)td.anchor[1], az = (double)td.anchor[2];
+  const uint32_t S = (uint32_t)e.item_pts;
+  uint32_t* const seeds = e.nn_seed + pr.pt_off;
+  const uint32_t* const word = (const uint32_t*)&e.st[0].gen;
+  if (tid == 0) sh.n_search = 0u;
+  uint32_t n_search = 0u;
+  int kept = 0;  // items held
+  for (int pass = 0; pass < e.prm.max_iter; ++pass) {
+    for (int o = 0; pass == 0 || o < kept; ++o) {
+      if (pass == 0) {
+        __syncthreads();  // (the last item's readers of sh.item)
+        if (tid == 0) {
+          const uint32_t c = atomicAdd(e.claim, 1u);
+          sh.item = c < pr.n_items ? (int)c : -1;
+        }
+        __syncthreads();
+        if (sh.item < 0) break;
+        if (tid == 0) s_item[o] = (uint16_t)sh.item;
+        kept = o + 1;
+      }
+      const int it = pass == 0 ? sh.item : (int)s_item[o];
+      const uint32_t first = (uint32_t)it * S, end = min(first + S, sd.n);
+      // the first queries, and what they start from, ahead of the transform
+      uint32_t j = first + (uint32_t)(tid >> 2);
+      float px = 0.f, py = 0.f, pz = 0.f;
+      uint32_t s0 = ~0u;
+      float4 t0 = make_float4(0.f, 0.f, 0.f, 0.f);
+      auto fetch = [&](uint32_t jj) {
+        s0 = ~0u;
+        if (jj < end) {
+          px = e.sx[sd.off + jj];
+          py = e.sy[sd.off + jj];
+          pz = e.sz[sd.off + jj];
+          if (pass > 0) s0 = seeds[jj];
+          if (s0 - g.pt_lo < g.n_pts) t0 = g.pts[s0];
+        }
+      };
+      fetch(j);
+      if (o == 0) {
+        if (w == 0) {
+          // bounded wait for this iteration's transform
+          uint32_t wv = load_relaxed(word);
+          int spins = 0;
+          while (!(wv & kFinishedBit) && (int)wv < pass) {
+            ++spins;
+            if (spins > kMaxSpins || ((spins & 255) == 0 && load_relaxed((const uint32_t*)e.error) != 0u)) {
+              if (lane == 0) atomicOr(e.error, 1);
+              break;
+            }
+            __builtin_amdgcn_s_sleep(1);
+            wv = load_relaxed(word);
+          }
+          const bool run = !(wv & kFinishedBit) && (int)wv == pass;
+          if (run && lane < 12) sh.m[lane] = (float)load_relaxed(&e.st[0].T[(lane & 3) * 4 + (lane >> 2)]);
+          if (lane == 0) {
+            sh.run = run ? 1 : 0;
+            sh.stride = run && load_relaxed(&e.st[0].stage) ? e.prm.coarse_stride : 1;
+          }
+        }
+        __syncthreads();
+        if (!sh.run) {
+          pass = e.prm.max_iter;  // finished (or the wait expired): leave both loops
+          break;
+        }
+      }
+      float m[12];
+#pragma unroll
+      for (int k = 0; k < 12; ++k)
+        m[k] = __builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__float_as_int(sh.m[k])));
+      const uint32_t stride = (uint32_t)sh.stride;
+      double acc[NS];
+#pragma unroll
+      for (int k = 0; k < NS; ++k) acc[k] = 0.0;
+      for (uint32_t base = first; base < end; base += kOneQueries) {
+        float qx, qy, qz;
+        int cx = 0, cy = 0, cz = 0;
+        apply_f32(m, px, py, pz, qx, qy, qz);
+        uint64_t key = kNoKey;
+        uint32_t where = 0u;
+        bool act = j < end && (stride == 1u || j % stride == 0u) && query_cell(g, qx, qy, qz, cx, cy, cz);
+        if (act && s0 - g.pt_lo < g.n_pts) {
+          key = nn_key(d2_f32(qx, qy, qz, t0.x, t0.y, t0.z), __float_as_int(t0.w));
+          where = s0;
+        }
+        // without a seed in reach the distance field may show that there is no
+        // match, and where the walk can pass over empty rows
+        int D = 0;
+        if (act && key_d2(key) > r2f && e.cell_dist) {
+          D = e.cell_dist[td.cell_off + ((uint32_t)cz * g.dy + cy) * g.dx + cx];
+          if (D >= td.skip_ring) act = false;
+        }
+        if (act) {
+          n_search += sub == 0 ? 1u : 0u;
+          const float bound = fminf(key_d2(key), r2f);
+          // (rows the quad would list: within 2^20, and not the unbounded first search)
+          const float side = sqrt_approx(bound) * g.inv_h;
+          if (key != kNoKey && side < 400.f) {
+            search_quad(g, qx, qy, qz, r2f, sub, key, where);
+          } else {
+            GlobalVis<8> vis;
+            vis.init(g.pts, qx, qy, qz);
+            vis.key = key;
+            vis.where = where;
+            search_global(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
+            key = vis.key;
+            where = vis.where & 0x7fffffffu;
+          }
+          if (sub == 0) {
+            if (key != kNoKey && where != s0) seeds[j] = where;
+            if (key_d2(key) <= r2f) {
+              const float4 c = where == s0 ? t0 : g.pts[where];
+              add_pair<MODE>(e, qx, qy, qz, c, where, key_d2(key), ax, ay, az, acc);
+            }
+          }
+        }
+        if (base + kOneQueries < end) {
+          j += kOneQueries;
+          fetch(j);
+        }
+      }
+      wave_totals<NS>(acc, sh, w, lane, false);
+      __syncthreads();
+      if (tid < NS) {
+        double s = sh.red[0][tid];
+        for (int ww = 1; ww < kWaves; ++ww) s += sh.red[ww][tid];
+        e.partials[(size_t)(pr.item_off + it) * NSUM_MAX + tid] = s;
+      }
+      __syncthreads();
+      if (tid == 0) {
+        const uint32_t prev = __hip_atomic_fetch_add(&e.done[0], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+        sh.last = (prev + 1u == (uint32_t)(pass + 1) * pr.n_items);
+        if (sh.last) acquire_agent();
+      }
+      __syncthreads();
+      if (sh.last) {
+        solve_problem<MODE, NS, WaveTileNone>(e, 0u, pr, td, pass, sh);
+        __syncthreads();
+      }
+    }
+    if (kept == 0) break;  // every item was taken before this workgroup started
+  }
+  n_search = wave_sum_u32(n_search);
+  if (lane == 0 && n_search) atomicAdd(e.queries_searched, (unsigned long long)n_search);
+}
+
 template <int MODE, bool TILE, int D, int W>
 static int blocks_per_cu_of() {
   int nb = 0;
@@ -943,9 +1218,24 @@ int icp_blocks_per_cu(int mode, int use_tile, int variant) {
                   : blocks_per_cu_of<RTR_MODE_POINT_TO_POINT, false, 4, 3>();
 }
 
+int icp_one_blocks_per_cu(int mode) {
+  int nb = 0;
+  const hipError_t rc = mode == RTR_MODE_POINT_TO_PLANE
+                            ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_icp_one<RTR_MODE_POINT_TO_PLANE>, kBlock, 0)
+                            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_icp_one<RTR_MODE_POINT_TO_POINT>, kBlock, 0);
+  return rc != hipSuccess || nb < 1 ? 1 : nb;
+}
+
 void launch_icp(const DevEngine& e, int grid_blocks, hipStream_t s) {
   hipLaunchKernelGGL(k_icp_init, dim3((e.n_prob + kBlock - 1) / kBlock), dim3(kBlock), 0, s, e);
   const dim3 g(grid_blocks), b(kBlock);
+  if (e.one) {
+    if (e.prm.mode == RTR_MODE_POINT_TO_PLANE)
+      hipLaunchKernelGGL(k_icp_one<RTR_MODE_POINT_TO_PLANE>, g, b, 0, s, e);
+    else
+      hipLaunchKernelGGL(k_icp_one<RTR_MODE_POINT_TO_POINT>, g, b, 0, s, e);
+    return;
+  }
   if (e.prm.mode == RTR_MODE_POINT_TO_PLANE) {
     if (e.use_tile)
       hipLaunchKernelGGL((k_icp<RTR_MODE_POINT_TO_PLANE, true, 8, 2>), g, b, 0, s, e);

@@ -395,3 +395,42 @@ def test_coarse_to_fine_ends_at_a_full_resolution_fixed_point():
                 nxt = oracle.icp(srcs[p], tgts[p], oracle.params(max_iter=1, r_max=0.05), guess=r["T"])
                 print(aa, p, it, r["coarse_iterations"], synth.rmse_between(nxt["T"], r["T"], srcs[p]))
                 assert synth.rmse_between(nxt["T"], r["T"], srcs[p]) < 2e-4
+
+
+@pytest.mark.parametrize("ns,nt,kw", [
+    (3, 50, {}), (63, 400, {}), (64, 400, {}), (65, 401, {}), (1000, 20000, {}), (33000, 9000, {}), (70001, 3000, {}),
+    (2000, 5000, dict(max_correspondence_distance=1e30)), (2000, 5000, dict(max_correspondence_distance=3.0)),
+    (2000, 5000, dict(max_correspondence_distance=0.004)), (3000, 5000, dict(anderson_memory=5)),
+    (3001, 5000, dict(coarse_stride=4, coarse_iterations=10)), (5000, 2, {}),
+    (3000, 8000, dict(mode=1)), (40000, 8000, dict(mode=1, coarse_stride=3, coarse_iterations=5))])
+def test_one_registration_kernel_equals_batch_engine(ns, nt, kw):
+    """The single API's kernel (items kept from the first iteration, four lanes
+    per query) against the batch engine's queue on the same problem: the same
+    correspondences every iteration, so the same iterations, states and
+    counts, and transforms that differ by the order of FP64 sums only."""
+    rng = np.random.default_rng(ns + nt)
+    tgt, src = synth.sample_many([synth.CHAIR, synth.CHAIR], [nt, ns], rng, 0.002)
+    src = synth.apply(synth.random_rigid(rng, 8.0, 0.03), src)
+    src[ns // 2] = np.nan
+    kw = dict(dict(max_iterations=30, max_correspondence_distance=0.05, transformation_epsilon=1e-8), **kw)
+    p = R.make_params(**kw)
+    icp = R.IterativeClosestPoint()
+    icp.set_params(p)
+    reg = R.BatchRegistration()
+    reg.set_params(p)
+    icp.setInputSource(src)
+    icp.setInputTarget(tgt)
+    reg.set_clouds([src], [tgt])
+    reg.set_problems([0], [0])
+    if kw.get("mode"):
+        icp.computeTargetNormals(10, (0.0, 0.0, 3.0))
+        reg.compute_target_normals(10, (0.0, 0.0, 3.0))
+    for rep in range(2):                      # the second align starts beside the first one's seeds
+        icp.align()
+        a, b = icp.getResult(), reg.align()[0]
+        for k in ("iterations", "state", "n_corr", "coarse_iterations"):
+            assert a[k] == b[k], k
+        # Anderson mixing amplifies the last bits of the sums; the plain iteration follows them
+        tol = 1e-6 if kw.get("anderson_memory") else 1e-10
+        assert np.abs(a["T"] - b["T"]).max() < tol and abs(a["mse"] - b["mse"]) <= tol * max(b["mse"], 1e-12)
+        assert icp.getTiming()["queries_searched"] == reg.timing()["queries_searched"]
