@@ -816,8 +816,10 @@ int Engine::compute_target_normals(int k, const float vp[3]) {
   launch_target_normals(e, k, vp[0], vp[1], vp[2], max_tgt_, stream_);
   RTR_HIP(hipGetLastError());
   RTR_HIP(hipStreamSynchronize(stream_));
+  // the kernel wrote the normals in cell order too: the grids just built serve
+  // the next align (rebuilding them cost 0.1 ms of a 366k-point target's 2.1)
   normals_valid_ = true;
-  grid_dirty_ = true;
+  grid_dirty_ = false;
   graph_dirty_ = true;
   return RTR_OK;
 }

@@ -1347,9 +1347,8 @@ struct KnnVisitor {
   float qx, qy, qz;
   int k, cnt;
   uint64_t kth;    // key[k - 1] once cnt == k
-  uint64_t* key;   // LDS, stride kNrmBlock
-  uint32_t* slot;  // LDS, stride kNrmBlock; nullptr keeps keys only (their low word is the point's original index)
-  __device__ void insert(const float4& t, uint32_t j) {
+  uint64_t* key;   // LDS, stride kNrmBlock (a key's low word is the point's original index)
+  __device__ void insert(const float4& t) {
     union {
       float f;
       int32_t i;
@@ -1360,11 +1359,9 @@ struct KnnVisitor {
     int pos = cnt < k ? cnt++ : k - 1;
     while (pos > 0 && kk < key[(pos - 1) * kNrmBlock]) {
       key[pos * kNrmBlock] = key[(pos - 1) * kNrmBlock];
-      if (slot) slot[pos * kNrmBlock] = slot[(pos - 1) * kNrmBlock];
       --pos;
     }
     key[pos * kNrmBlock] = kk;
-    if (slot) slot[pos * kNrmBlock] = j;
     if (cnt == k) kth = key[(k - 1) * kNrmBlock];
   }
   __device__ void scan(uint32_t b, uint32_t e) {
@@ -1374,9 +1371,9 @@ struct KnnVisitor {
 #pragma unroll
       for (int u = 0; u < 4; ++u) t[u] = pts[j + u];
 #pragma unroll
-      for (int u = 0; u < 4; ++u) insert(t[u], j + u);
+      for (int u = 0; u < 4; ++u) insert(t[u]);
     }
-    for (; j < e; ++j) insert(pts[j], j);
+    for (; j < e; ++j) insert(pts[j]);
   }
   __device__ float bound() const { return cnt < k ? 3.4e38f : key_d2(kth); }
   // the judge's list interface: reset, size, and the keys in ascending order
@@ -1499,51 +1496,53 @@ __device__ void jacobi3(double* a, double* V) {
 // One thread per cell-sorted target point: exact k nearest (ordered by
 // (d2, index), the point itself included), FP64 two-pass covariance, the
 // eigenvector of the smallest eigenvalue, flipped towards the viewpoint
-// (pcl::NormalEstimation + flipNormalTowardsViewpoint semantics).
-__global__ __launch_bounds__(kNrmBlock) void k_target_normals(DevEngine e, int k, float vpx,
-                                                              float vpy, float vpz,
-                                                              float* nrm_raw) {
-  // k-NN lists in dynamic LDS sized for k (as in k_judge)
+// (pcl::NormalEstimation + flipNormalTowardsViewpoint semantics).  The lists as
+// in k_judge: registers for k = 20, else dynamic LDS sized for k, keys only.
+// 330k points, k = 20: 0.97 -> 0.34 ms, the insertions into LDS lists having
+// been a chain of shifts at LDS latency; the points behind the keys are read
+// once more for the covariance, from L2.
+template <int K>
+__global__ __launch_bounds__(kNrmBlock) __attribute__((amdgpu_waves_per_eu(3))) void k_target_normals(
+    DevEngine e, int k, float vpx, float vpy, float vpz, float* nrm_raw) {
   extern __shared__ uint64_t s_dyn[];
-  uint64_t* const s_key = s_dyn;
-  uint32_t* const s_slot = reinterpret_cast<uint32_t*>(s_dyn + (size_t)k * kNrmBlock);
   const TargetDesc td = e.tgts[blockIdx.y];
   const GridView g = grid_of(e, td);
   const uint32_t base = e.cell_start[td.cell_off];
+  const float* const raw = e.tgt_raw + 3 * (size_t)td.raw_off;
   for (uint32_t j0 = blockIdx.x * blockDim.x; j0 < td.n_valid; j0 += gridDim.x * blockDim.x) {
     const uint32_t j = j0 + threadIdx.x;
     if (j >= td.n_valid) continue;
     const float4 q = e.tgt_sorted[base + j];
-    KnnVisitor v;
+    typename std::conditional<K == 0, KnnVisitor, KnnRegList<(K > 0 ? K : 1)>>::type v;
     v.pts = e.tgt_sorted;
     v.qx = q.x;
     v.qy = q.y;
     v.qz = q.z;
-    v.k = k;
-    v.cnt = 0;
-    v.key = s_key + threadIdx.x;
-    v.slot = s_slot + threadIdx.x;
+    if constexpr (K == 0) {
+      v.k = k;
+      v.key = s_dyn + threadIdx.x;
+    }
+    v.reset();
     ring_walk(g, q.x, q.y, q.z, FLT_MAX, v);
     double nv[3] = {__builtin_nan(""), __builtin_nan(""), __builtin_nan("")};
-    if (v.cnt >= 3) {
+    const int nn = v.size();
+    if (nn >= 3) {
       double mean[3] = {0, 0, 0};
-#pragma unroll 4
-      for (int i = 0; i < v.cnt; ++i) {
-        const float4 p = e.tgt_sorted[v.slot[i * kNrmBlock]];
-        mean[0] += p.x;
-        mean[1] += p.y;
-        mean[2] += p.z;
-      }
-      for (int a = 0; a < 3; ++a) mean[a] /= v.cnt;
+      v.for_each([&](uint64_t key) {
+        const float* p = raw + 3 * (size_t)(uint32_t)key;
+        mean[0] += p[0];
+        mean[1] += p[1];
+        mean[2] += p[2];
+      });
+      for (int a = 0; a < 3; ++a) mean[a] /= nn;
       double C[9] = {0, 0, 0, 0, 0, 0, 0, 0, 0};
-#pragma unroll 4
-      for (int i = 0; i < v.cnt; ++i) {
-        const float4 p = e.tgt_sorted[v.slot[i * kNrmBlock]];
-        const double d[3] = {p.x - mean[0], p.y - mean[1], p.z - mean[2]};
+      v.for_each([&](uint64_t key) {
+        const float* p = raw + 3 * (size_t)(uint32_t)key;
+        const double d[3] = {p[0] - mean[0], p[1] - mean[1], p[2] - mean[2]};
         for (int r = 0; r < 3; ++r)
           for (int c = 0; c < 3; ++c) C[r * 3 + c] += d[r] * d[c];
-      }
-      for (int i = 0; i < 9; ++i) C[i] /= v.cnt;
+      });
+      for (int i = 0; i < 9; ++i) C[i] /= nn;
       double V[9];
       jacobi3(C, V);
       int mi = 0;
@@ -1559,12 +1558,7 @@ __global__ __launch_bounds__(kNrmBlock) void k_target_normals(DevEngine e, int k
         nv[2] = -nv[2];
       }
     }
-    union {
-      float f;
-      int32_t i;
-    } w;
-    w.f = q.w;
-    float* o = nrm_raw + 3 * ((size_t)td.raw_off + (uint32_t)w.i);
+    float* o = nrm_raw + 3 * ((size_t)td.raw_off + (uint32_t)__float_as_int(q.w));
     o[0] = (float)nv[0];
     o[1] = (float)nv[1];
     o[2] = (float)nv[2];
@@ -1578,10 +1572,13 @@ void launch_target_normals(const DevEngine& e, int k, float vpx, float vpy, floa
   if (k > kMaxK) k = kMaxK;
   unsigned bx = (unsigned)((max_tgt_pts + kNrmBlock - 1) / kNrmBlock);
   if (bx < 1) bx = 1;
-  if (bx > 1024) bx = 1024;
-  const size_t lds = (size_t)k * kNrmBlock * (sizeof(uint64_t) + sizeof(uint32_t));
-  hipLaunchKernelGGL(k_target_normals, dim3(bx, e.n_tgt), dim3(kNrmBlock), lds, s, e, k, vpx, vpy,
-                     vpz, const_cast<float*>(e.tgt_nrm_raw));
+  if (bx > 1u << 16) bx = 1u << 16;
+  float* const raw = const_cast<float*>(e.tgt_nrm_raw);
+  if (k == 20)
+    hipLaunchKernelGGL(k_target_normals<20>, dim3(bx, e.n_tgt), dim3(kNrmBlock), 0, s, e, k, vpx, vpy, vpz, raw);
+  else
+    hipLaunchKernelGGL(k_target_normals<0>, dim3(bx, e.n_tgt), dim3(kNrmBlock),
+                       (size_t)k * kNrmBlock * sizeof(uint64_t), s, e, k, vpx, vpy, vpz, raw);
 }
 
 
@@ -1645,7 +1642,6 @@ __global__ __launch_bounds__(kNrmBlock) __attribute__((amdgpu_waves_per_eu(3))) 
     if constexpr (K == 0) {
       v.k = k;
       v.key = s_key + threadIdx.x;
-      v.slot = nullptr;
     }
     v.reset();
     // A query whose cell's distance-field value reaches skip_ring has no

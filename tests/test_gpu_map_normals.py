@@ -27,6 +27,32 @@ def test_normals_match_oracle():
     assert np.all(np.isfinite(n_gpu))
 
 
+@pytest.mark.parametrize("k", [3, 19, 20, 21, 32])
+@pytest.mark.parametrize("n", [2, 20, 129, 3000])
+def test_normals_for_every_list_form(k, n):
+    """k = 20 keeps its neighbour lists in registers, every other k in LDS.
+    Both sum the same k points in ascending (distance, index) order in FP64,
+    so away from ties of the eigenvalues only the final float32 rounding is
+    left: 1e-5 covers it with a relative eigenvalue gap down to 1e-10.  Fewer
+    than three points give NaN.  The align that follows uses the same grid."""
+    rng = np.random.default_rng(100 * k + n)
+    tgt = rng.uniform(-1, 1, (n, 3)).astype(np.float32) * np.float32([1.0, 0.7, 0.02])
+    icp = R.IterativeClosestPointWithNormals()
+    icp.setInputSource(tgt)
+    icp.setInputTarget(tgt)
+    icp.computeTargetNormals(k, (0.0, 0.0, 2.0))
+    got = icp.getTargetNormals()
+    ref, _ = oracle.normals(tgt, k, vp=(0.0, 0.0, 2.0))
+    if n < 3:
+        assert np.isnan(got).all()
+        return
+    assert np.abs(got - ref).max() < 1e-5
+    icp.setMaxCorrespondenceDistance(0.5)
+    icp.setMaximumIterations(3)
+    icp.align()
+    assert np.abs(icp.getFinalTransformation() - np.eye(4)).max() < 1e-6
+
+
 def test_point_to_plane_matches_oracle():
     src, tgt, T_gt = synth.config1_pair(1)
     nrm, _ = oracle.normals(tgt, 20, vp=(0.0, 0.0, 2.0))
