@@ -59,7 +59,7 @@ Engine::~Engine() {
     if (e) (void)hipEventDestroy(e);
   DevBuf* bufs[] = {&tgt_raw_, &tgt_nrm_raw_, &tgt_sorted_, &tgt_nrm_sorted_, &cell_count_,
                     &cell_start_, &cell_id_, &cell_rank_, &cell_dist_, &cell_dist_tmp_, &tgt_desc_, &bbox_tmp_, &src_raw_, &sx_, &sy_, &sz_, &perm_,
-                    &bin_count_, &bin_start_, &bin_id_, &bin_rank_, &src_desc_, &prob_desc_, &state_,
+                    &bin_count_, &bin_start_, &bin_id_, &bin_rank_, &src_key_, &src_desc_, &prob_desc_, &state_,
                     &guesses_, &items_buf_, &partials_, &done_, &counters_, &scan_tmp_,
                     &out_i32_, &out_f32_, &out_T_, &hist_, &aa_, &nn_seed_, &tline_};
   for (DevBuf* b : bufs) b->release();
@@ -198,6 +198,7 @@ int Engine::set_clouds(int n_src, const float* const* src, const size_t* ns, con
     RTR_TRY(perm_.ensure(st * 4));
     RTR_TRY(bin_id_.ensure(st * 4));
     RTR_TRY(bin_rank_.ensure(st * 4));
+    RTR_TRY(src_key_.ensure(st * 8));
     RTR_TRY(bin_count_.ensure((size_t)n_bins_ * 4));
     RTR_TRY(bin_start_.ensure((size_t)n_bins_ * 4));
   }
@@ -474,6 +475,7 @@ DevEngine Engine::dev_view() const {
   e.bin_start = bin_start_.as<uint32_t>();
   e.bin_id = bin_id_.as<uint32_t>();
   e.bin_rank = bin_rank_.as<uint32_t>();
+  e.src_key = src_key_.as<uint64_t>();
   e.n_bins_total = n_bins_;
   e.probs = prob_desc_.as<Problem>();
   e.n_prob = (int)probs_.size();
@@ -561,7 +563,7 @@ int Engine::grid_blocks() const {
 int Engine::enqueue_build() {
   DevEngine e = dev_view();
   launch_target_grid(e, max_tgt_, max_cells_, stream_);
-  launch_source_sort(e, max_src_, (uint32_t)src_total_, stream_);
+  launch_source_sort(e, max_src_, stream_);
   RTR_HIP(hipGetLastError());
   return RTR_OK;
 }

@@ -40,6 +40,7 @@ struct DevEngine {
   uint32_t* bin_start;
   uint32_t* bin_id;          // per raw source point
   uint32_t* bin_rank;        // per raw source point: its slot within its bin
+  uint64_t* src_key;         // per source point, bin by bin: (bin, fine Morton code, original index)
   uint32_t n_bins_total;
   // problems and the work queue
   const Problem* probs;
@@ -82,7 +83,7 @@ void launch_exclusive_scan(const uint32_t* in, uint32_t* out, uint32_t n, uint32
                            hipStream_t s);
 size_t scan_tmp_words(uint32_t n);
 void launch_target_grid(const DevEngine& e, int max_tgt_pts, int max_cells, hipStream_t s);
-void launch_source_sort(const DevEngine& e, int max_src_pts, uint32_t src_total, hipStream_t s);
+void launch_source_sort(const DevEngine& e, int max_src_pts, hipStream_t s);
 void launch_icp(const DevEngine& e, int grid_blocks, hipStream_t s);
 int icp_blocks_per_cu(int mode, int use_tile, int variant);
 int icp_one_blocks_per_cu(int mode);

@@ -434,3 +434,32 @@ def test_one_registration_kernel_equals_batch_engine(ns, nt, kw):
         tol = 1e-6 if kw.get("anderson_memory") else 1e-10
         assert np.abs(a["T"] - b["T"]).max() < tol and abs(a["mse"] - b["mse"]) <= tol * max(b["mse"], 1e-12)
         assert icp.getTiming()["queries_searched"] == reg.timing()["queries_searched"]
+
+
+def test_source_order_of_crowded_bins():
+    """The source sort ranks each point among its bin's keys: one point, bins
+    of 7, 1023, 1024 (the largest ordered by position), 1025 and 3000 points
+    (by index), non-finite points and a plain cloud, all in one engine.  Every
+    point is placed once (correspondences of each, bit-exact), and the order,
+    and with it every sum, is the same from build to build."""
+    rng = np.random.default_rng(17)
+    far = np.float32([[1.0, 1.0, 1.0]])
+    srcs = []
+    for n in (1, 7, 1023, 1024, 1025, 3000):
+        crowd = (0.01 * rng.random((n, 3))).astype(np.float32)
+        srcs.append(crowd if n == 1 else np.concatenate([crowd, far]))
+    srcs.append(rng.random((5000, 3)).astype(np.float32))
+    srcs[-1][::97] = np.nan
+    tgt = np.concatenate([rng.random((4000, 3)), 0.012 * rng.random((2000, 3))]).astype(np.float32)
+    runs = []
+    for rep in range(2):
+        b = R.BatchRegistration()
+        b.set_params(R.make_params(max_iterations=1, max_correspondence_distance=0.3, min_correspondences=1))
+        b.set_clouds(srcs, [tgt])
+        b.set_problems(np.arange(len(srcs)), np.zeros(len(srcs), np.int64))
+        runs.append([r["T"].copy() for r in b.align()])
+        for p, s in enumerate(srcs):
+            idx, d2 = b.last_correspondences(p)
+            i_ref, d_ref = oracle.nn_brute(s, tgt, 0.3)
+            assert np.array_equal(idx, i_ref) and np.array_equal(d2, d_ref), p
+    assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(*runs))
