@@ -84,6 +84,9 @@ __device__ __forceinline__ GridView grid_of(const DevEngine& e, const TargetDesc
 // before e.fine_from, the fine ones (kFinePts) from then on.  The items a
 // problem completes up to and including pass k (its done count then).
 __device__ __forceinline__ bool fine_pass(const DevEngine& e, int pass) { return pass >= e.fine_from; }
+__device__ __forceinline__ uint32_t item_points(const DevEngine& e, int pass) {
+  return fine_pass(e, pass) ? (uint32_t)kFinePts : (uint32_t)e.item_pts;
+}
 __device__ __forceinline__ uint32_t items_of(const Problem& pr, bool fine) { return fine ? pr.n_fitems : pr.n_items; }
 __device__ __forceinline__ uint32_t first_item_of(const Problem& pr, bool fine) {
   return fine ? pr.fitem_off : pr.item_off;
@@ -182,6 +185,7 @@ struct IcpShared {
   int stride;             // this iteration's source stride (coarse stage: > 1)
   int stage_reset;        // the solve moved the problem to all source points
   int item;
+  int cnt;                // items taken together
   int run;
   int stop;
   int last;
@@ -501,6 +505,14 @@ __device__ __forceinline__ void wave_totals(const double* acc, Sh& sh, int w, in
   }
 }
 
+// ... and the four waves' sums in a fixed order
+template <class Sh>
+__device__ __forceinline__ double wave_sums(const Sh& sh, int k) {
+  double s = sh.red[0][k];
+  for (int w = 1; w < kWaves; ++w) s += sh.red[w][k];
+  return s;
+}
+
 // A copy of a wave-uniform value in scalar registers: loads of descriptors
 // through a uniform address come back in vector registers, and the pointers
 // derived from them would otherwise hold vector registers through the walk.
@@ -516,10 +528,11 @@ __device__ __forceinline__ T scalar_copy(const T& v) {
 }
 
 template <int MODE, int NS, bool TILE, class TileT, int DEPTH>
-__device__ void process_item(const DevEngine& e, int it, int pass, IcpShared<NS, TileT>& sh) {
+__device__ void process_items(const DevEngine& e, int it, int cnt, int pass, IcpShared<NS, TileT>& sh) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   TileT& tl = sh.tile[w];
   it = __builtin_amdgcn_readfirstlane(it);
+  cnt = __builtin_amdgcn_readfirstlane(cnt);
   const uint2 itm = scalar_copy(e.items[it]);
   const uint32_t p = itm.x;
   const Problem pr = scalar_copy(e.probs[p]);
@@ -536,7 +549,8 @@ __device__ void process_item(const DevEngine& e, int it, int pass, IcpShared<NS,
   const double ay = (double)__builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__float_as_int(sh.anchor[1])));
   const double az = (double)__builtin_bit_cast(float, __builtin_amdgcn_readfirstlane(__float_as_int(sh.anchor[2])));
   uint32_t n_search = 0u;
-  const uint32_t end = min(itm.y + (fine_pass(e, pass) ? (uint32_t)kFinePts : (uint32_t)e.item_pts), sd.n);
+  const uint32_t ipts = item_points(e, pass);
+  const uint32_t end = min(itm.y + (uint32_t)cnt * ipts, sd.n);
   constexpr bool kCompact = !TILE && DEPTH == 4;
   // Search seeds (global walks only): every searched query stores its
   // nearest neighbour's slot, and the next iteration starts from it.  The
@@ -655,21 +669,29 @@ __device__ void process_item(const DevEngine& e, int it, int pass, IcpShared<NS,
       // Moment phase: the walks above keep no moment sums live (their
       // registers go to the gathers in flight); the chunk's correspondences
       // are re-read from LDS in query order, each query's transform and
-      // squared distance recomputed exactly as the walk computed them.
-      double acc[NS];
+      // squared distance recomputed exactly as the walk computed them.  The
+      // sums are those of each item by itself, whatever was walked with it.
+      for (uint32_t i0 = 0; i0 < cn; i0 += ipts) {
+        const uint32_t i1 = min(i0 + ipts, cn);
+        double acc[NS];
 #pragma unroll
-      for (int k = 0; k < NS; ++k) acc[k] = 0.0;
-      for (uint32_t o = tid; o < cn; o += kBlock) {
-        const uint32_t slot = sh.qseed[o];
-        if (slot == ~0u) continue;
-        const uint32_t sj = sd.off + chunk + o;
-        float qx, qy, qz;
-        apply_f32(m, e.sx[sj], e.sy[sj], e.sz[sj], qx, qy, qz);
-        const float4 c = g.pts[slot];
-        add_pair<MODE>(e, qx, qy, qz, c, slot, d2_f32(qx, qy, qz, c.x, c.y, c.z), ax, ay, az, acc);
+        for (int k = 0; k < NS; ++k) acc[k] = 0.0;
+        for (uint32_t o = i0 + tid; o < i1; o += kBlock) {
+          const uint32_t slot = sh.qseed[o];
+          if (slot == ~0u) continue;
+          const uint32_t sj = sd.off + chunk + o;
+          float qx, qy, qz;
+          apply_f32(m, e.sx[sj], e.sy[sj], e.sz[sj], qx, qy, qz);
+          const float4 c = g.pts[slot];
+          add_pair<MODE>(e, qx, qy, qz, c, slot, d2_f32(qx, qy, qz, c.x, c.y, c.z), ax, ay, az, acc);
+        }
+        wave_totals<NS>(acc, sh, w, lane, cnt == 1 && chunk != itm.y);
+        __syncthreads();  // (also: the next chunk rewrites the lists)
+        if (cnt > 1) {
+          if (tid < NS) e.partials[(size_t)(it + (int)(i0 / ipts)) * NSUM_MAX + tid] = wave_sums(sh, tid);
+          __syncthreads();
+        }
       }
-      wave_totals<NS>(acc, sh, w, lane, chunk != itm.y);
-      __syncthreads();  // the next chunk rewrites the lists
     }
   }
   double acc[NS];
@@ -819,15 +841,11 @@ __device__ void process_item(const DevEngine& e, int it, int pass, IcpShared<NS,
   // wave totals (DPP row sums), then the four waves in a fixed order
   if (!kCompact) wave_totals<NS>(acc, sh, w, lane, false);
   __syncthreads();
-  if (tid < NS) {
-    double s = sh.red[0][tid];
-    for (int ww = 1; ww < kWaves; ++ww) s += sh.red[ww][tid];
-    e.partials[(size_t)it * NSUM_MAX + tid] = s;
-  }
+  if (cnt == 1 && tid < NS) e.partials[(size_t)it * NSUM_MAX + tid] = wave_sums(sh, tid);
   __syncthreads();
   if (tid == 0) {
-    const uint32_t prev = __hip_atomic_fetch_add(&e.done[p], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
-    sh.last = (prev + 1u == done_through(e, pr, pass));
+    const uint32_t prev = __hip_atomic_fetch_add(&e.done[p], (uint32_t)cnt, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+    sh.last = (prev + (uint32_t)cnt == done_through(e, pr, pass));
     if (sh.last) acquire_agent();
   }
   __syncthreads();
@@ -857,40 +875,65 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
     // polling the work queue stretch the last problems' iterations.  They
     // leave between passes, holding no claimed item, and one workgroup per CU
     // stays, so every remaining item is still claimed.
+    const bool fine = fine_pass(e, pass);
+    const uint32_t* const qoff = fine ? e.fxcd_off : e.xcd_off;
+    uint32_t take = 1u;           // items per claim
+    uint32_t nit = 0u, nend = 0u; // (thread 0) what is left of the last claim
+    uint32_t* nctr = nullptr;     // its counter, and where the counter's queue starts
+    uint32_t nq = 0u;
     if (tid == 0) {
       const uint32_t done = load_relaxed(e.problems_done);
       sh.stop = (done >= (uint32_t)e.n_prob) || (load_relaxed((const uint32_t*)e.error) != 0u) ||
                 ((int)blockIdx.x >= e.retire_from && done + e.retire_active >= (uint32_t)e.n_prob);
+      // Items per claim: as many as fill a chunk while the items still in play
+      // give every workgroup a claim, one by one as they run out.  A claim
+      // costs the queue's atomic, the transform's acquire, five barriers and
+      // the list whatever its size: 256 pairs from the identity on 256-point
+      // items 47.1 -> 36.0 ms, on 512-point ones 38.8 -> 35.7 (chunks of 2048
+      // queries, LDS and all: 46 ms, the last claims of a pass hold up the next).
+      if (!TILE && DEPTH == 4) {
+        const uint32_t most = (uint32_t)kChunk / item_points(e, pass);  // 0 for larger items
+        const uint32_t left = (uint32_t)((uint64_t)(qoff[kXcds] - qoff[0]) * (uint32_t)(e.n_prob - (int)done) / (uint32_t)e.n_prob);
+        take = max(1u, min(most, left / gridDim.x));
+      }
     }
     __syncthreads();
     if (sh.stop) break;
     for (;;) {
       if (tid == 0) {
         // own XCD's queue first (L2 locality), then steal from the others
-        int it = e.n_items;
+        int it = e.n_items, cnt = 1;
         const int x0 = (int)(blockIdx.x % kXcds);
-        const bool fine = fine_pass(e, pass);
-        const uint32_t* qoff = fine ? e.fxcd_off : e.xcd_off;
-        for (int t = 0; t < kXcds; ++t) {
-          const int x = (x0 + t) % kXcds;
-          const uint32_t cnt = qoff[x + 1] - qoff[x];
-          uint32_t* ctr = &e.claim[(size_t)(pass * kXcds + x) * e.claim_stride];
-          if (cnt == 0u || __hip_atomic_load(ctr, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) >= cnt) continue;
-          const uint32_t c = atomicAdd(ctr, 1u);
-          if (c < cnt) {
-            it = (int)(qoff[x] + c);
-            const uint32_t p = e.items[it].x;
-            if (load_relaxed((const uint32_t*)&e.st[p].gen) & kFinishedBit) {
-              // a finished problem: its remaining items of this pass (contiguous
-              // in this queue) are skipped in one step, and the claim goes on
-              const Problem& pr = e.probs[p];
-              atomicMax(ctr, first_item_of(pr, fine) + items_of(pr, fine) - qoff[x]);
-              it = e.n_items;
-              t = -1;  // rescan the queues from the own XCD's
-              continue;
-            }
-            break;
+        for (;;) {
+          if (nit < nend) {
+            const uint32_t p = e.items[nit].x;
+            const Problem& pr = e.probs[p];
+            const uint32_t pend = first_item_of(pr, fine) + items_of(pr, fine);
+            const bool finished = load_relaxed((const uint32_t*)&e.st[p].gen) & kFinishedBit;
+            it = (int)nit;
+            nit = min(nend, pend);
+            cnt = (int)nit - it;
+            if (!finished) break;
+            // a finished problem: its remaining items of this pass (contiguous
+            // in this queue) are skipped in one step, and the claim goes on
+            if (nit == nend) atomicMax(nctr, pend - nq);
+            it = e.n_items;
+            continue;
           }
+          for (int t = 0; t < kXcds && nit >= nend; ++t) {
+            const int x = (x0 + t) % kXcds;
+            const uint32_t n = qoff[x + 1] - qoff[x];
+            uint32_t* ctr = &e.claim[(size_t)(pass * kXcds + x) * e.claim_stride];
+            if (n == 0u || load_relaxed(ctr) >= n) continue;
+            const uint32_t c = atomicAdd(ctr, take);
+            if (c < n) {
+              nit = qoff[x] + c;
+              nend = qoff[x] + min(c + take, n);
+              nctr = ctr;
+              nq = qoff[x];
+            }
+          }
+          if (nit >= nend) break;  // nothing left in this pass
         }
         int run = 0;
         if (it < e.n_items) {
@@ -924,12 +967,13 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
           }
         }
         sh.item = it;
+        sh.cnt = cnt;
         sh.run = run;
       }
       __syncthreads();
       const int it = sh.item;
       if (it >= e.n_items) break;
-      if (sh.run) process_item<MODE, NS, TILE, TileT, DEPTH>(e, it, pass, sh);
+      if (sh.run) process_items<MODE, NS, TILE, TileT, DEPTH>(e, it, sh.cnt, pass, sh);
       __syncthreads();
     }
   }
@@ -1174,11 +1218,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
       }
       wave_totals<NS>(acc, sh, w, lane, false);
       __syncthreads();
-      if (tid < NS) {
-        double s = sh.red[0][tid];
-        for (int ww = 1; ww < kWaves; ++ww) s += sh.red[ww][tid];
-        e.partials[(size_t)(pr.item_off + it) * NSUM_MAX + tid] = s;
-      }
+      if (tid < NS) e.partials[(size_t)(pr.item_off + it) * NSUM_MAX + tid] = wave_sums(sh, tid);
       __syncthreads();
       if (tid == 0) {
         const uint32_t prev = __hip_atomic_fetch_add(&e.done[0], 1u, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);

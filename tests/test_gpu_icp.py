@@ -463,3 +463,31 @@ def test_source_order_of_crowded_bins():
             i_ref, d_ref = oracle.nn_brute(s, tgt, 0.3)
             assert np.array_equal(idx, i_ref) and np.array_equal(d2, d_ref), p
     assert all(np.array_equal(x, y, equal_nan=True) for x, y in zip(*runs))
+
+
+@pytest.mark.parametrize("item_pts,fine_from", [(256, 0), (512, 0), (768, 0), (1024, 0), (1280, 0), (256, 3), (512, 2)])
+def test_items_taken_together_keep_their_own_sums(item_pts, fine_from):
+    """A claim takes several work items while plenty are left; each still sums
+    its own points.  So a problem's result is the same, bit for bit, among
+    400 others (claims of up to a chunk) and by itself (one item each), for
+    sizes around the items' and the chunk's edges."""
+    rng = np.random.default_rng(item_pts + fine_from)
+    sizes = [1, 255, 256, 257, 511, 513, 1023, 1024, 1025, 2047, 2049, 3071, 3500]
+    ns = sizes + [int(n) for n in rng.integers(1800, 2200, 400)]
+    tgt = synth.sample_many([synth.CHAIR], [5000], rng, 0.002)[0]
+    srcs = [synth.apply(synth.random_rigid(rng, 8.0, 0.02), tgt[rng.integers(0, len(tgt), n)]) for n in ns]
+    p = R.make_params(max_iterations=12, max_correspondence_distance=0.05, min_correspondences=1)
+
+    def run(idx):
+        b = R.BatchRegistration()
+        b.set_tuning(item_pts=item_pts, fine_from=fine_from)
+        b.set_params(p)
+        b.set_clouds([srcs[i] for i in idx], [tgt])
+        b.set_problems(np.arange(len(idx)), np.zeros(len(idx), np.int64))
+        return b.align()
+
+    many = run(range(len(ns)))
+    for i in range(len(sizes)):
+        one = run([i])[0]
+        assert one["iterations"] == many[i]["iterations"] and one["n_corr"] == many[i]["n_corr"], sizes[i]
+        assert np.array_equal(one["T"], many[i]["T"]) and one["mse"] == many[i]["mse"], sizes[i]
