@@ -919,7 +919,9 @@ int Engine::last_correspondences(int prob, int32_t* idx, float* d2) {
   RTR_HIP(hipMemcpyAsync(&st, state_.as<ProblemState>() + prob, sizeof(st), hipMemcpyDeviceToHost, stream_));
   const Problem pr = probs_[prob];
   TargetDesc td;
+  uint32_t base = 0;  // the target's first slot: the points of the targets before it that are finite
   RTR_HIP(hipMemcpyAsync(&td, tgt_desc_.as<TargetDesc>() + pr.tgt, sizeof(td), hipMemcpyDeviceToHost, stream_));
+  RTR_HIP(hipMemcpyAsync(&base, cell_start_.as<uint32_t>() + tgts_[pr.tgt].cell_off, 4, hipMemcpyDeviceToHost, stream_));
   RTR_HIP(hipStreamSynchronize(stream_));
   if (st.iter < 1) {
     set_error("problem %d ran no iteration", prob);
@@ -936,7 +938,7 @@ int Engine::last_correspondences(int prob, int32_t* idx, float* d2) {
   RTR_HIP(hipMemcpyAsync(y.data(), sy_.as<float>() + sd.off, n * 4, hipMemcpyDeviceToHost, stream_));
   RTR_HIP(hipMemcpyAsync(z.data(), sz_.as<float>() + sd.off, n * 4, hipMemcpyDeviceToHost, stream_));
   if (td.n_valid)
-    RTR_HIP(hipMemcpyAsync(tp.data(), tgt_sorted_.as<float4>() + td.raw_off, (size_t)td.n_valid * sizeof(float4),
+    RTR_HIP(hipMemcpyAsync(tp.data(), tgt_sorted_.as<float4>() + base, (size_t)td.n_valid * sizeof(float4),
                            hipMemcpyDeviceToHost, stream_));
   const size_t hoff = ((size_t)prob * (prm_.max_iterations + 1) + (size_t)(st.iter - 1)) * 12;
   RTR_HIP(hipMemcpyAsync(rows.data(), hist_.as<float>() + hoff, 12 * sizeof(float), hipMemcpyDeviceToHost, stream_));
@@ -946,7 +948,7 @@ int Engine::last_correspondences(int prob, int32_t* idx, float* d2) {
     const uint32_t o = perm[j];
     idx[o] = -1;
     d2[o] = INFINITY;
-    const uint32_t s = slot[j] - td.raw_off;
+    const uint32_t s = slot[j] - base;
     if (s >= td.n_valid) continue;
     float qx, qy, qz;
     apply_f32(rows.data(), x[j], y[j], z[j], qx, qy, qz);

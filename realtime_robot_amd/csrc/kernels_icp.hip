@@ -70,7 +70,8 @@ __device__ __forceinline__ GridView grid_of(const DevEngine& e, const TargetDesc
   g.dy = td.dy;
   g.dz = td.dz;
   g.n_pts = td.n_valid;
-  g.pt_lo = td.raw_off;
+  // (not its raw offset: targets before it may hold points that are not finite)
+  g.pt_lo = __builtin_amdgcn_readfirstlane(e.cell_start[td.cell_off]);
   g.ox = td.ox;
   g.oy = td.oy;
   g.oz = td.oz;
@@ -213,31 +214,46 @@ constexpr uint64_t kNoKey = 0x7f800000ffffffffull;
 template <int D>
 struct GlobalVis {
   const float4* pts;
+  uint32_t last;  // the target's last D points start here
   float qx, qy, qz;
   uint64_t key;
   uint32_t where;
-  __device__ __forceinline__ void init(const float4* p, float x, float y, float z) {
-    pts = p;
+  __device__ __forceinline__ void init(const GridView& g, float x, float y, float z) {
+    pts = g.pts;
+    last = g.pt_lo + g.n_pts - D;
     qx = x;
     qy = y;
     qz = z;
     key = kNoKey;
     where = 0u;
   }
+  __device__ __forceinline__ void take(float d, float w, uint32_t slot) {
+    const uint64_t k = nn_key(d, __float_as_int(w));
+    if (k < key) {
+      key = k;
+      where = slot | 0x80000000u;
+    }
+  }
   // D (4 or 8) independent loads in flight per step: the gathers are
   // latency-bound, and the deeper variant needs the registers of a kernel
-  // that runs 2 waves per SIMD.  A range's last step loads its last point
-  // again in place of the missing ones (the same key twice changes nothing),
-  // so a short range costs one round of loads, not one per point.  A step
-  // whose smallest distance exceeds the best so far, most of them once the
-  // walk is seeded, ends there; else its points' keys are compared.
+  // that runs 2 waves per SIMD.  A step always takes D neighbouring slots, one
+  // address and D offsets, whatever is left of the range (moved back at the
+  // target's end, for targets of at least D points): points beyond the range
+  // are points of the target all the same, and a short range costs one round
+  // of loads, not one per point.  A step whose smallest distance exceeds the
+  // best so far, most of them once the walk is seeded, ends there; else its
+  // points' keys are compared.  (A minimum and a 64-bit address for each load,
+  // and the first index read late: 256 pairs 36.0 -> 34.0 ms without them.)
   __device__ __forceinline__ void scan(uint32_t b, uint32_t e) {
-    if (b >= e) return;
-    const uint32_t last = e - 1;
     for (uint32_t j = b; j < e; j += D) {
+      const uint32_t j0 = min(j, last);
+      const float4* const p = pts + j0;
       float4 t[D];
 #pragma unroll
-      for (int u = 0; u < D; ++u) t[u] = pts[min(j + u, last)];
+      for (int u = 0; u < D; ++u) t[u] = p[u];
+      // (the first index arrives with its point: left to itself the compiler
+      // loads it where it is compared, behind the branch, and waits again)
+      asm("" : "+v"(t[0].w));
       float d[D];
 #pragma unroll
       for (int u = 0; u < D; ++u) d[u] = d2_f32(qx, qy, qz, t[u].x, t[u].y, t[u].z);
@@ -246,14 +262,15 @@ struct GlobalVis {
       for (int u = 1; u < D; ++u) m = fminf(m, d[u]);
       if (m <= key_d2(key)) {
 #pragma unroll
-        for (int u = 0; u < D; ++u) {
-          const uint64_t k = nn_key(d[u], __float_as_int(t[u].w));
-          if (k < key) {
-            key = k;
-            where = min(j + u, last) | 0x80000000u;
-          }
-        }
+        for (int u = 0; u < D; ++u) take(d[u], t[u].w, j0 + u);
       }
+    }
+  }
+  // every point of a target too small for scan()
+  __device__ __forceinline__ void scan_all(const GridView& g) {
+    for (uint32_t j = g.pt_lo; j < g.pt_lo + g.n_pts; ++j) {
+      const float4 t = pts[j];
+      take(d2_f32(qx, qy, qz, t.x, t.y, t.z), t.w, j);
     }
   }
   __device__ __forceinline__ float bound() const { return key_d2(key); }
@@ -328,7 +345,7 @@ __device__ __forceinline__ void walk_block_global(const GridView& g, float qx, f
 // gathers (a row's cell bounds, then its points), and VALU issue about 40 % of
 // the cycles.  The shell-by-shell walk tested every row of every shell,
 // (2k + 1)^2 of them, to find the few a seeded query needs; the ball's rows
-// need no test beyond the first one out of reach on each side.  256 pairs from
+// need no test beyond the first one out of reach on each side.  Then 256 pairs from
 // the identity 66.3 -> 50.0 ms, 32 pairs x 8 starts 59 -> 31-35 ms, one 10k x
 // 20k pair 3.2 -> 2.2 ms, the learned call of 256 pairs 11.3 -> 9.6 ms
 // (identical results).  Measured and left out: two or four rows' bounds
@@ -338,6 +355,10 @@ __device__ __forceinline__ void walk_block_global(const GridView& g, float qx, f
 template <int DEPTH>
 __device__ __forceinline__ void search_global(const GridView& g, float qx, float qy, float qz, int cx, int cy, int cz,
                                               int D, float r2f, GlobalVis<DEPTH>& vis) {
+  if (g.n_pts < (uint32_t)DEPTH) {
+    vis.scan_all(g);
+    return;
+  }
   if (fminf(vis.bound(), r2f) < 1.0e30f) {
     walk_ball(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
     return;
@@ -650,7 +671,7 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
           const int D = sh.qd[o];
           ++n_search;
           GlobalVis<DEPTH> vis;
-          vis.init(g.pts, qx, qy, qz);
+          vis.init(g, qx, qy, qz);
           const uint32_t s0 = sh.qseed[o];
           if (s0 - g.pt_lo < g.n_pts) vis.seed(s0);
           search_global(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
@@ -725,7 +746,7 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
     }
     if (act) ++n_search;
     GlobalVis<DEPTH> vis;
-    vis.init(g.pts, qx, qy, qz);
+    vis.init(g, qx, qy, qz);
     if (act && s0 - g.pt_lo < g.n_pts) vis.seed(s0);
     bool staged = false;
     int X0 = 0, Y0 = 0, Z0 = 0, NY = 1, W1 = 1, nrows = 0;
@@ -771,7 +792,10 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
       }
     }
     if (act) {
-      if (!TILE) {
+      const bool few = TILE && g.n_pts < (uint32_t)DEPTH;
+      if (few) {
+        vis.scan_all(g);
+      } else if (!TILE) {
         search_global(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
       } else if (!blk) {
         // block known empty: only the outer rings
@@ -814,7 +838,7 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
       } else {
         walk_block_global(g, qx, qy, qz, cx, cy, cz, r2f, vis);
       }
-      if (TILE) walk_far(g, qx, qy, qz, cx, cy, cz, r2f, vis, k0);
+      if (TILE && !few) walk_far(g, qx, qy, qz, cx, cy, cz, r2f, vis, k0);
       if (seeds && vis.key != kNoKey && (vis.where & 0x7fffffffu) != s0) seeds[j] = vis.where & 0x7fffffffu;
       if (key_d2(vis.key) <= r2f) {
         float4 c;
@@ -1196,7 +1220,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
             search_quad(g, qx, qy, qz, r2f, sub, key, where);
           } else {
             GlobalVis<8> vis;
-            vis.init(g.pts, qx, qy, qz);
+            vis.init(g, qx, qy, qz);
             vis.key = key;
             vis.where = where;
             search_global(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);

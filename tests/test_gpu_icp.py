@@ -491,3 +491,44 @@ def test_items_taken_together_keep_their_own_sums(item_pts, fine_from):
         one = run([i])[0]
         assert one["iterations"] == many[i]["iterations"] and one["n_corr"] == many[i]["n_corr"], sizes[i]
         assert np.array_equal(one["T"], many[i]["T"]) and one["mse"] == many[i]["mse"], sizes[i]
+
+
+@pytest.mark.parametrize("use_tile,blocks_per_cu", [(0, 0), (0, 2), (0, 4), (1, 0), (1, 2)])
+@pytest.mark.parametrize("rmax", [0.4, 1e30])
+def test_targets_around_the_search_step(use_tile, blocks_per_cu, rmax):
+    """The search reads 4 or 8 neighbouring slots a step, moved back at the
+    target's end, and smaller targets whole: targets of 1 to 17 points between
+    targets with non-finite points, so that a slot read from a neighbour, or
+    counted from the raw offsets, would show.  Correspondences of the second
+    iteration (seeded) bit-exact; the tiled search, which records none, by the
+    first iteration's count and error."""
+    rng = np.random.default_rng(5)
+    tgts = []
+    for n in (3, 1, 2, 4, 5, 7, 8, 9, 12, 17, 40):
+        t = rng.random((n, 3)).astype(np.float32)
+        if n in (3, 9, 40):
+            t[1] = np.nan
+        tgts.append(t)
+    srcs = [rng.random((300, 3)).astype(np.float32) for _ in tgts]
+    b = R.BatchRegistration()
+    b.set_tuning(use_tile=use_tile, blocks_per_cu=blocks_per_cu)
+    b.set_params(R.make_params(max_iterations=1 if use_tile else 2, max_correspondence_distance=rmax,
+                               min_correspondences=1, transformation_epsilon=0.0, euclidean_fitness_epsilon=-1.0))
+    b.set_clouds(srcs, tgts)
+    b.set_problems(np.arange(len(tgts)), np.arange(len(tgts)))
+    if use_tile:
+        for p, r in enumerate(b.align()):
+            _, d_ref = oracle.nn_brute(srcs[p], tgts[p], rmax)
+            d_ref = d_ref[np.isfinite(d_ref)].astype(np.float64)
+            assert r["n_corr"] == len(d_ref) and abs(r["mse"] - d_ref.mean()) <= 1e-12 * d_ref.mean()
+        return
+    for rep in range(2):                      # again beside the first launch's seeds
+        res = b.align()
+        for p, r in enumerate(res):
+            if r["iterations"] < 1:
+                continue
+            T = np.eye(4)
+            T[:3] = b.history(p, 3)[r["iterations"] - 1]
+            idx, d2 = b.last_correspondences(p)
+            i_ref, d_ref = oracle.nn_brute(oracle.transform(T, srcs[p]), tgts[p], rmax)
+            assert np.array_equal(idx, i_ref) and np.array_equal(d2, d_ref), (p, len(tgts[p]))
