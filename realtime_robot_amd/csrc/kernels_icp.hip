@@ -611,7 +611,9 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
       }
       __syncthreads();
       {
-        // The walk list: class by class, each class in query order.  Wave w
+        // The walk list: class by class, each class in query order, the longest
+        // walks first, so that the waves end the list on its short ones (256
+        // pairs 34.0 -> 32.0 ms, 32 x 8 starts 30.5 -> 28.7).  Wave w
         // lists the classes of its quarter of the chunk (kSegs runs of 64
         // queries): counts per class first, then each wave writes from the
         // offset of its class in the earlier classes and earlier waves.
@@ -633,7 +635,7 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
         __syncthreads();
         uint32_t nl = 0;  // the list's length so far (classes below cls, all waves)
 #pragma unroll
-        for (int cls = 1; cls <= kQueryClasses; ++cls) {
+        for (int cls = kQueryClasses; cls >= 1; --cls) {
           uint32_t off = nl;
           for (int v = 0; v < kWaves; ++v) {
             const uint32_t n = sh.ccount[v][cls - 1];
