@@ -548,7 +548,7 @@ __device__ __forceinline__ T scalar_copy(const T& v) {
   return out;
 }
 
-template <int MODE, int NS, bool TILE, class TileT, int DEPTH>
+template <int MODE, int NS, bool TILE, class TileT, int DEPTH, int WALK>
 __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, IcpShared<NS, TileT>& sh) {
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6;
   TileT& tl = sh.tile[w];
@@ -672,7 +672,7 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
           query_cell(g, qx, qy, qz, cx, cy, cz);
           const int D = sh.qd[o];
           ++n_search;
-          GlobalVis<DEPTH> vis;
+          GlobalVis<WALK> vis;
           vis.init(g, qx, qy, qz);
           const uint32_t s0 = sh.qseed[o];
           if (s0 - g.pt_lo < g.n_pts) vis.seed(s0);
@@ -881,7 +881,7 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
 }
 
 template <int MODE, bool TILE, int DEPTH, int WAVES>
-// Point-to-point with 4-deep gathers asks for at least 3 waves per SIMD
+// Point-to-point with 4-deep gathers (8-deep in its compacted walk) asks for at least 3 waves per SIMD
 // (<= 168 VGPRs): the gathers of the ring walk are latency-bound, so
 // resident waves are what hides them; a variant asks for 4 (<= 128 VGPRs,
 // its few spills outside the walks) for launches tuned to 4 workgroups per
@@ -891,6 +891,10 @@ template <int MODE, bool TILE, int DEPTH, int WAVES>
 // sums, runs 2 waves per SIMD and is always 8-deep.
 __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
   constexpr int NS = MODE == RTR_MODE_POINT_TO_POINT ? SUM_P2P_COUNT : SUM_P2L_COUNT;
+  // Points per step of the compacted walk: 8 at 3 waves per SIMD (256 pairs 32.0
+  // -> 29.7 ms, 32 x 8 starts 28.7 -> 27.3; 6 measured 30.3 and 27.6, 12 as 8),
+  // 4 where 128 registers would spill the wider step.
+  constexpr int WALK = !TILE && DEPTH == 4 && WAVES == 3 ? 8 : DEPTH;
   using TileT = typename std::conditional<TILE, WaveTile, WaveTileNone>::type;
   __shared__ IcpShared<NS, TileT> sh;
   const int tid = threadIdx.x;
@@ -999,7 +1003,7 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
       __syncthreads();
       const int it = sh.item;
       if (it >= e.n_items) break;
-      if (sh.run) process_items<MODE, NS, TILE, TileT, DEPTH>(e, it, sh.cnt, pass, sh);
+      if (sh.run) process_items<MODE, NS, TILE, TileT, DEPTH, WALK>(e, it, sh.cnt, pass, sh);
       __syncthreads();
     }
   }
