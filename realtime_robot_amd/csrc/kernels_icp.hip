@@ -17,10 +17,11 @@
 // queue and steals from the others when it is empty, and a claim that lands
 // on a finished problem skips that problem's remaining items of the pass.
 //
-// Two search variants: the throughput variant (4 gathers in flight per lane,
-// 3 or 4 waves/SIMD) classifies an item's queries first and walks them from a
-// compacted list grouped by distance-field class; the latency variant (8
-// gathers in flight, 2 waves/SIMD) walks each 64-query round directly.  With
+// Two search variants: the throughput variant (3 or 4 waves/SIMD) takes up to
+// a chunk of items at a time, classifies their queries first and walks them
+// from a compacted list grouped by distance-field class; the latency variant (8
+// gathers in flight, 2 waves/SIMD) walks each 64-query round directly.  One
+// registration by itself has a kernel of its own, k_icp_one.  With
 // Anderson acceleration on, the solving workgroup also extrapolates the next
 // iterate (geom.hpp).
 #include <hip/hip_runtime.h>
@@ -881,8 +882,8 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
 }
 
 template <int MODE, bool TILE, int DEPTH, int WAVES>
-// Point-to-point with 4-deep gathers (8-deep in its compacted walk) asks for at least 3 waves per SIMD
-// (<= 168 VGPRs): the gathers of the ring walk are latency-bound, so
+// Point-to-point with 4-deep gathers (8-deep in its compacted walk) asks for at
+// least 3 waves per SIMD (<= 168 VGPRs): the walk's gathers are latency-bound, so
 // resident waves are what hides them; a variant asks for 4 (<= 128 VGPRs,
 // its few spills outside the walks) for launches tuned to 4 workgroups per
 // CU.  The 8-deep variant keeps more gathers in flight per wave and runs 2
