@@ -486,6 +486,7 @@ DevEngine Engine::dev_view() const {
                                                                                           : nullptr;
   e.aa = prm_.anderson_memory > 0 ? aa_.as<double>() : nullptr;
   e.nn_seed = (pt_total_ > 0 && pt_total_ <= 0xffffffffull) ? nn_seed_.as<uint32_t>() : nullptr;
+  e.n_seeds = e.nn_seed && !tune_.use_tile ? (size_t)pt_total_ : 0;
   e.items = items_buf_.as<uint2>();
   e.n_items = (int)items_.size();
   e.item_pts = (int)item_points();

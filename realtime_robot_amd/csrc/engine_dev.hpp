@@ -53,6 +53,7 @@ struct DevEngine {
   double* aa;                // n_prob * kAndersonStride: acceleration state (null when off)
   uint32_t* nn_seed;         // per problem and sorted source point (at Problem::pt_off): cell-sorted
                              // slot of its last nearest neighbour, the next search's seed (nullable)
+  size_t n_seeds;            // its length (0 where the launch keeps no seeds)
   const uint2* items;        // (problem, first sorted source point)
   int n_items;
   int item_pts;              // points per item

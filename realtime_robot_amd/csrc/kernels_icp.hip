@@ -26,6 +26,7 @@
 // iterate (geom.hpp).
 #include <hip/hip_runtime.h>
 
+#include <algorithm>
 #include <cfloat>
 #include <type_traits>
 
@@ -98,8 +99,13 @@ __device__ __forceinline__ uint32_t done_through(const DevEngine& e, const Probl
   return (uint32_t)e.fine_from * pr.n_items + (uint32_t)(pass + 1 - e.fine_from) * pr.n_fitems;
 }
 
+// The problems' state, and no search seeds: a launch's seeds are its own.  A
+// point that is not searched in the first iteration (no match in reach, or the
+// coarse stage passes it over) would otherwise start from what an earlier
+// launch left, and pass for a correspondence of this one.
 __global__ void k_icp_init(DevEngine e) {
   const int p = blockIdx.x * blockDim.x + threadIdx.x;
+  for (size_t i = (size_t)p; i < e.n_seeds; i += (size_t)gridDim.x * blockDim.x) e.nn_seed[i] = ~0u;
   if (p >= e.n_prob) return;
   ProblemState& S = e.st[p];
   for (int k = 0; k < 16; ++k) S.T[k] = e.guesses ? e.guesses[16 * (size_t)p + k] : ((k % 5 == 0) ? 1.0 : 0.0);
@@ -579,8 +585,8 @@ __device__ void process_items(const DevEngine& e, int it, int cnt, int pass, Icp
   // transform moves little between iterations, so the seed's distance is
   // close to the nearest one: it trims the block's rows before their bounds
   // are loaded and stops the outer walk early.  Any slot of this target gives
-  // a valid bound, so a seed is only range-checked, and the first iteration
-  // of a launch (slots from an earlier launch) starts without one.
+  // a valid bound, so a seed is only range-checked.  k_icp_init cleared them
+  // all, so the first iteration need not look.
   uint32_t* const seeds = !TILE && e.nn_seed ? e.nn_seed + pr.pt_off : nullptr;
   const int stride = sh.stride;  // coarse stage: every stride-th source point
   const bool seeded = seeds && pass > 0;
@@ -1032,6 +1038,11 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
 // the solve take 6); 30k x 366k points point-to-plane: the launch 1.0 -> 0.7 ms.
 // ---------------------------------------------------------------------------
 constexpr int kOneQueries = kBlock / 4;  // queries a workgroup searches at a time
+// Four lanes also search a query that has no seed (it had no match so far) when
+// r_max is within this many cells: most find none, so all rows of the ball have
+// to be seen, and four lanes see them four times as fast (r_max is 4 cells of
+// an untuned grid: 2k x 10k points 1.13 -> 0.93 ms a call, 10k x 20k 1.55 -> 1.19).
+constexpr float kQuadUnseeded = 8.f;
 
 template <int I>
 __device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
@@ -1221,9 +1232,10 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
         if (act) {
           n_search += sub == 0 ? 1u : 0u;
           const float bound = fminf(key_d2(key), r2f);
-          // (rows the quad would list: within 2^20, and not the unbounded first search)
+          // (rows the quad would list: within 2^20; and without a seed the ball of
+          // r_max, whose rows the quad does not take nearest first, small)
           const float side = sqrt_approx(bound) * g.inv_h;
-          if (key != kNoKey && side < 400.f) {
+          if (side < (key != kNoKey ? 400.f : kQuadUnseeded)) {
             search_quad(g, qx, qy, qz, r2f, sub, key, where);
           } else {
             GlobalVis<8> vis;
@@ -1298,7 +1310,9 @@ int icp_one_blocks_per_cu(int mode) {
 }
 
 void launch_icp(const DevEngine& e, int grid_blocks, hipStream_t s) {
-  hipLaunchKernelGGL(k_icp_init, dim3((e.n_prob + kBlock - 1) / kBlock), dim3(kBlock), 0, s, e);
+  const size_t seed_blocks = std::min<size_t>((e.n_seeds + 4 * kBlock - 1) / (4 * kBlock), 2048);
+  const unsigned init_blocks = std::max((unsigned)((e.n_prob + kBlock - 1) / kBlock), (unsigned)seed_blocks);
+  hipLaunchKernelGGL(k_icp_init, dim3(init_blocks), dim3(kBlock), 0, s, e);
   const dim3 g(grid_blocks), b(kBlock);
   if (e.one) {
     if (e.prm.mode == RTR_MODE_POINT_TO_PLANE)

@@ -532,3 +532,28 @@ def test_targets_around_the_search_step(use_tile, blocks_per_cu, rmax):
             idx, d2 = b.last_correspondences(p)
             i_ref, d_ref = oracle.nn_brute(oracle.transform(T, srcs[p]), tgts[p], rmax)
             assert np.array_equal(idx, i_ref) and np.array_equal(d2, d_ref), (p, len(tgts[p]))
+
+
+def test_correspondences_of_an_iteration_on_the_subsample():
+    """An iteration of the coarse stage searches every fourth point: the other
+    points have no correspondence in it, whatever an earlier launch on the same
+    handle, or the memory before it, left in the search seeds."""
+    rng = np.random.default_rng(23)
+    tgt, src = synth.sample_many([synth.CHAIR, synth.CHAIR], [6000, 3001], rng, 0.002)
+    src = synth.apply(synth.random_rigid(rng, 3.0, 0.01), src)
+    b = R.BatchRegistration()
+    b.set_params(R.make_params(max_iterations=2, max_correspondence_distance=0.05))
+    b.set_clouds([src], [tgt])
+    b.set_problems([0], [0])
+    b.align()
+    assert (b.last_correspondences(0)[0] >= 0).all()
+    for guess in (np.eye(4), synth.random_rigid(rng, 1.0, 0.001)):
+        b.set_params(R.make_params(max_iterations=1, max_correspondence_distance=0.05, coarse_stride=4,
+                                   coarse_iterations=5))
+        r = b.align([guess])[0]
+        idx, d2 = b.last_correspondences(0)
+        i_ref, d_ref = oracle.nn_brute(oracle.transform(guess, src), tgt, 0.05)
+        got = idx >= 0
+        assert r["n_corr"] == got.sum() <= (len(src) + 3) // 4
+        assert np.array_equal(idx[got], i_ref[got]) and np.array_equal(d2[got], d_ref[got])
+        assert np.isinf(d2[~got]).all()
