@@ -420,6 +420,61 @@ RTR_HD void walk_ball(const GridView& g, float qx, float qy, float qz, int cx, i
   }
 }
 
+// The rows (y, z) of cells that the ball of squared radius B about a query can
+// meet, as one list in which lanes take a row each: all rows of a box, found as
+// walk_ball finds a row's cells.  False when a side has more than kBallSide
+// rows.  The limit is on the box as it is, margin included: a target far from
+// the origin on small cells has a margin of many cells.  It keeps row r's
+// division by ny exact: r is below 2^20, so the quotient's error, under r / ny
+// 2^-22, stays below the 0.5 / ny that separate (r + 0.5) / ny from a whole
+// number.
+struct BallRows {
+  int y0, ny, z0, nz;
+};
+constexpr int kBallSide = 1023;
+// k_icp_one's four lanes also search a query that has no seed (it had no match
+// so far) when r_max is within this many cells: most find none, so all rows of
+// the ball have to be seen, and four lanes see them four times as fast (r_max
+// is 4 cells of an untuned grid: 2k x 10k points 1.13 -> 0.93 ms a call, 10k x
+// 20k 1.55 -> 1.19).
+constexpr float kQuadUnseeded = 8.f;
+
+RTR_HD bool ball_rows(const GridView& g, float qy, float qz, float B, BallRows& o) {
+  const float w = sqrt_approx(B) * 1.00001f + 2.0f * g.margin;
+  const float ya = ((qy - w) - g.oy) * g.inv_h, yb = ((qy + w) - g.oy) * g.inv_h;
+  const float za = ((qz - w) - g.oz) * g.inv_h, zb = ((qz + w) - g.oz) * g.inv_h;
+  const int y1 = (int)floorf(fminf(fmaxf(yb, -1.f), 1.0e9f)), z1 = (int)floorf(fminf(fmaxf(zb, -1.f), 1.0e9f));
+  o.y0 = (int)fminf(fmaxf(ya, 0.f), 1.0e9f);
+  o.z0 = (int)fminf(fmaxf(za, 0.f), 1.0e9f);
+  o.ny = (y1 < g.dy - 1 ? y1 : g.dy - 1) - o.y0 + 1;
+  o.nz = (z1 < g.dz - 1 ? z1 : g.dz - 1) - o.z0 + 1;
+  return o.ny <= kBallSide && o.nz <= kBallSide;
+}
+
+// Row r of the list (r in [0, ny nz)): its y and z.  inv_ny = 1 / ny.
+RTR_HD void ball_row(const BallRows& o, float inv_ny, int r, int& y, int& z) {
+  const int dz = (int)(((float)r + 0.5f) * inv_ny);
+  y = o.y0 + (r - dz * o.ny);
+  z = o.z0 + dz;
+}
+
+// The points of row (y, z) within what B leaves of the ball: slots [b, e).
+RTR_HD void ball_row_range(const GridView& g, float qx, float qy, float qz, float B, int y, int z, uint32_t& b,
+                           uint32_t& e) {
+  b = e = 0u;
+  const float gy = slab_gap(qy, g.oy, g.h, g.margin, y, y), gz = slab_gap(qz, g.oz, g.h, g.margin, z, z);
+  const float rem = B - (gy * gy + gz * gz);
+  if (!(rem >= 0.f)) return;
+  const float w = sqrt_approx(rem) * 1.00001f + 2.0f * g.margin;
+  const int xa = (int)fminf(fmaxf(((qx - w) - g.ox) * g.inv_h, 0.f), 1.0e9f);
+  const int x1 = (int)floorf(fminf(fmaxf(((qx + w) - g.ox) * g.inv_h, -1.f), 1.0e9f));
+  const int xb = x1 < g.dx - 1 ? x1 : g.dx - 1;
+  if (xa > xb) return;
+  const uint32_t row = ((uint32_t)z * g.dy + y) * g.dx;
+  b = g.cell_start[row + (uint32_t)xa];
+  e = g.cell_start[row + (uint32_t)xb + 1u];
+}
+
 // Distance-field parameters for a grid of cell edge h: a query whose cell is
 // at Chebyshev distance >= R from every occupied cell is at least
 // (R - 1) * h - margin from every target point; skip_ring is the smallest R

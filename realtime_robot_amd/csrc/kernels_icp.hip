@@ -1038,11 +1038,6 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
 // the solve take 6); 30k x 366k points point-to-plane: the launch 1.0 -> 0.7 ms.
 // ---------------------------------------------------------------------------
 constexpr int kOneQueries = kBlock / 4;  // queries a workgroup searches at a time
-// Four lanes also search a query that has no seed (it had no match so far) when
-// r_max is within this many cells: most find none, so all rows of the ball have
-// to be seen, and four lanes see them four times as fast (r_max is 4 cells of
-// an untuned grid: 2k x 10k points 1.13 -> 0.93 ms a call, 10k x 20k 1.55 -> 1.19).
-constexpr float kQuadUnseeded = 8.f;
 
 template <int I>
 __device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
@@ -1063,40 +1058,23 @@ __device__ __forceinline__ void quad_min(uint64_t& key, uint32_t& where) {
 
 // Four lanes search one query from its seed: key (and where, its slot) hold the
 // seed's on entry, equal in the four lanes, and the nearest point's on return.
-// Every cell that can hold a point within min(seed, r2f) is in the rows
-// [y0, y1] x [z0, z1]; each row is cut as in walk_ball, with the bound of the
-// rows before it.  All four lanes are active or none.
+// Every cell that can hold a point within min(seed, r2f) is in the rows of box;
+// each row is cut as in walk_ball, with the bound of the rows before it.  All
+// four lanes are active or none.
 __device__ __forceinline__ void search_quad(const GridView& g, float qx, float qy, float qz, float r2f, int sub,
-                                            uint64_t& key, uint32_t& where) {
+                                            const BallRows& box, uint64_t& key, uint32_t& where) {
+  if (box.ny <= 0 || box.nz <= 0) return;
   float B = fminf(key_d2(key), r2f) * 1.000004f;
-  const float w = sqrt_approx(B) * 1.00001f + 2.0f * g.margin;
-  auto lo_of = [&](float q, float o) { return (int)fminf(fmaxf(((q - w) - o) * g.inv_h, 0.f), 1.0e9f); };
-  auto hi_of = [&](float q, float o, int n) {
-    return min((int)floorf(fminf(fmaxf(((q + w) - o) * g.inv_h, -1.f), 1.0e9f)), n - 1);
-  };
-  const int y0 = lo_of(qy, g.oy), ny = hi_of(qy, g.oy, g.dy) - y0 + 1;
-  const int z0 = lo_of(qz, g.oz), nz = hi_of(qz, g.oz, g.dz) - z0 + 1;
-  if (ny <= 0 || nz <= 0) return;
-  const int nrows = ny * nz;
-  const float inv_ny = 1.0f / (float)ny;
+  const int nrows = box.ny * box.nz;
+  const float inv_ny = 1.0f / (float)box.ny;
   for (int r0 = 0; r0 < nrows; r0 += 4) {
     const int r = r0 + sub;
-    // r / ny: exact, the callers keep nrows below 2^20 (the quotient's error
-    // stays far below the half that separates it from a whole number)
-    const int dz = (int)(((float)r + 0.5f) * inv_ny);
-    const int y = y0 + (r - dz * ny), z = z0 + dz;
-    const float gy = slab_gap(qy, g.oy, g.h, g.margin, y, y), gz = slab_gap(qz, g.oz, g.h, g.margin, z, z);
-    const float rem = B - (gy * gy + gz * gz);
     uint32_t b = 0u, n = 0u;
-    if (r < nrows && rem >= 0.f) {
-      const float wx = sqrt_approx(rem) * 1.00001f + 2.0f * g.margin;
-      const int xa = (int)fminf(fmaxf(((qx - wx) - g.ox) * g.inv_h, 0.f), 1.0e9f);
-      const int xb = min((int)floorf(fminf(fmaxf(((qx + wx) - g.ox) * g.inv_h, -1.f), 1.0e9f)), g.dx - 1);
-      if (xa <= xb) {
-        const uint32_t row = ((uint32_t)z * g.dy + y) * g.dx;
-        b = g.cell_start[row + (uint32_t)xa];
-        n = g.cell_start[row + (uint32_t)xb + 1u] - b;
-      }
+    if (r < nrows) {
+      int y, z;
+      ball_row(box, inv_ny, r, y, z);
+      ball_row_range(g, qx, qy, qz, B, y, z, b, n);
+      n -= b;
     }
     // the four rows' points as one list: point t is pts[t + base of its row]
     const uint32_t n1 = quad_bcast<0>(n), n2 = n1 + quad_bcast<1>(n), n3 = n2 + quad_bcast<2>(n);
@@ -1232,11 +1210,12 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
         if (act) {
           n_search += sub == 0 ? 1u : 0u;
           const float bound = fminf(key_d2(key), r2f);
-          // (rows the quad would list: within 2^20; and without a seed the ball of
-          // r_max, whose rows the quad does not take nearest first, small)
+          // (without a seed the ball of r_max, whose rows the quad does not take
+          // nearest first, has to be small)
           const float side = sqrt_approx(bound) * g.inv_h;
-          if (side < (key != kNoKey ? 400.f : kQuadUnseeded)) {
-            search_quad(g, qx, qy, qz, r2f, sub, key, where);
+          BallRows box;
+          if (side < (key != kNoKey ? 400.f : kQuadUnseeded) && ball_rows(g, qy, qz, bound * 1.000004f, box)) {
+            search_quad(g, qx, qy, qz, r2f, sub, box, key, where);
           } else {
             GlobalVis<8> vis;
             vis.init(g, qx, qy, qz);

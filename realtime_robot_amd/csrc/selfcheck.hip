@@ -14,6 +14,41 @@
 
 using rtr::set_error;
 
+namespace rtr {
+
+// k_icp_one's search of a seeded query, four rows at a time, one after the
+// other: false when its rows are more than it takes.  A row outside the grid or
+// a range outside the target sets *bad.
+static bool quad_search(const GridView& g, float r2f, NNCountVisitor& v, bool* bad) {
+  BallRows box;
+  float B = std::fmin(v.bound(), r2f) * 1.000004f;
+  if (!ball_rows(g, v.qy, v.qz, B, box)) return false;
+  if (box.ny <= 0 || box.nz <= 0) return true;
+  const int nrows = box.ny * box.nz;
+  for (int r0 = 0; r0 < nrows; r0 += 4) {
+    uint32_t b[4] = {0, 0, 0, 0}, e[4] = {0, 0, 0, 0};
+    for (int u = 0; u < 4 && r0 + u < nrows; ++u) {
+      int y, z;
+      ball_row(box, 1.0f / (float)box.ny, r0 + u, y, z);
+      if (y < box.y0 || y >= box.y0 + box.ny || z < box.z0 || z >= box.z0 + box.nz || y < 0 || y >= g.dy || z < 0 ||
+          z >= g.dz) {
+        *bad = true;
+        return true;
+      }
+      ball_row_range(g, v.qx, v.qy, v.qz, B, y, z, b[u], e[u]);
+      if (b[u] > e[u] || e[u] > g.n_pts) {
+        *bad = true;
+        return true;
+      }
+    }
+    for (int u = 0; u < 4; ++u) v.scan(b[u], e[u]);
+    B = std::fmin(v.bound(), r2f) * 1.000004f;
+  }
+  return true;
+}
+
+}  // namespace rtr
+
 extern "C" {
 
 // ---------------------------------------------------------------------------
@@ -130,10 +165,23 @@ int rtr_selfcheck_nn_stats(const float* tgt, size_t nt, const float* q, size_t n
     // every other query starts from a seed, some point of the target, as the
     // kernel's queries start from their last nearest neighbour
     int cx, cy, cz;
-    if ((i & 1) && query_cell(g, v.qx, v.qy, v.qz, cx, cy, cz)) {
-      const uint32_t s0 = (uint32_t)((i * 2654435761ull) % nv);
-      v.scan(s0, s0 + 1);
-      v.ranges = v.cands = 0;
+    if (query_cell(g, v.qx, v.qy, v.qz, cx, cy, cz)) {
+      if (i & 1) {
+        const uint32_t s0 = (uint32_t)((i * 2654435761ull) % nv);
+        v.scan(s0, s0 + 1);
+        v.ranges = v.cands = 0;
+      }
+      // k_icp_one's search from the same start has to find the same point
+      NNCountVisitor one = v, walk = v;
+      bool bad = false;
+      if (((i & 1) || std::sqrt(r2f) * g.inv_h < kQuadUnseeded) && quad_search(g, r2f, one, &bad)) {
+        ring_walk_dt(g, da.data(), skip_ring, v.qx, v.qy, v.qz, r2f, walk);
+        const bool found = key_d2(walk.best.key) <= r2f;
+        if (bad || (found ? one.best.key != walk.best.key : key_d2(one.best.key) <= r2f)) {
+          set_error("query %zu: the row list and the walk differ", i);
+          return RTR_ERR_DEVICE;
+        }
+      }
     }
     ring_walk_dt(g, da.data(), skip_ring, v.qx, v.qy, v.qz, r2f, v);
     NNBest b = v.best;

@@ -193,6 +193,22 @@ def test_host_ball_walk_matches_brute_force(shape, rmax):
         assert np.array_equal(i1, i2) and np.array_equal(d1, d2)
 
 
+def test_host_row_list_far_from_the_origin():
+    """A target a kilometre out on cells far below its coordinates' spacing: the
+    grid's margin alone spans 2000 rows to each side of a query, and the box more
+    rows than the list's division is exact for (numbers of 2^23 and above), so
+    the list has to refuse it.  The search hook runs the list beside the walk wherever it
+    takes a query, and reports a row or a range outside the grid."""
+    rng = np.random.default_rng(2)
+    t = (1000.0 + rng.uniform(0, 0.015, (400, 3))).astype(np.float32)
+    t[:, 0] = 1000.0
+    q = (1000.0 + rng.uniform(0.0065, 0.0085, (8, 3))).astype(np.float32)
+    q[:, 0] = 1000.0
+    i1, d1 = R.selfcheck_nn(t, q, 4e-6, 0.0015)
+    i2, d2 = oracle.nn_brute(q, t, 0.0015)
+    assert np.array_equal(i1, i2) and np.array_equal(d1, d2)
+
+
 def test_host_solver_matches_oracle():
     from scipy.spatial.transform import Rotation
     rng = np.random.default_rng(4)
