@@ -47,6 +47,8 @@ int Engine::init() {
   RTR_HIP(hipStreamCreateWithFlags(&stream_, hipStreamNonBlocking));
   for (auto& e : ev_) RTR_HIP(hipEventCreate(&e));
   RTR_HIP(hipDeviceGetAttribute(&cu_count_, hipDeviceAttributeMultiprocessorCount, device_));
+  RTR_HIP(hipDeviceGetAttribute(&wall_khz_, hipDeviceAttributeWallClockRate, device_));
+  if (wall_khz_ <= 0) wall_khz_ = 100000;
   return RTR_OK;
 }
 
@@ -501,6 +503,7 @@ DevEngine Engine::dev_view() const {
   // their own: spinning workgroups poll the flag while others claim
   e.problems_done = ctr;
   e.error = reinterpret_cast<int*>(ctr + 32);
+  e.wait_ticks = 10000ull * (unsigned long long)wall_khz_;  // ten seconds
   e.queries_searched = reinterpret_cast<unsigned long long*>(ctr + 64);
   e.claim = ctr + 96;
   e.claim_stride = claim_stride();
@@ -888,9 +891,7 @@ int Engine::timeline(int prob, uint64_t* stamps, int cap, int* n_out, double* ti
     set_error("timeline of %d stamps, buffer holds %d", n, cap);
     return RTR_ERR_CAPACITY;
   }
-  int khz = 0;
-  RTR_HIP(hipDeviceGetAttribute(&khz, hipDeviceAttributeWallClockRate, device_));
-  *tick_ns = khz > 0 ? 1e6 / (double)khz : 0.0;
+  *tick_ns = 1e6 / (double)wall_khz_;
   RTR_HIP(hipMemcpyAsync(stamps, tline_.as<uint64_t>() + (size_t)prob * prm_.max_iterations * 2,
                          (size_t)n * sizeof(uint64_t), hipMemcpyDeviceToHost, stream_));
   RTR_HIP(hipStreamSynchronize(stream_));

@@ -137,6 +137,7 @@ class Engine {
   bool results_valid_ = false;  // states/grids hold a completed align of the current layout
   bool normals_valid_ = false;
   int cu_count_ = 0;
+  int wall_khz_ = 0;  // rate of the device's wall clock
   rtr_params prm_;
   TuneParams tune_;
   rtr_timing timing_;

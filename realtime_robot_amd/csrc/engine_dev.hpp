@@ -72,6 +72,7 @@ struct DevEngine {
   uint32_t* done;            // per problem: items finished so far
   uint32_t* problems_done;
   int* error;                // nonzero: a bounded wait expired
+  unsigned long long wait_ticks;  // the bound, in ticks of the device's wall clock
   unsigned long long* queries_searched;  // nearest-neighbour searches of the launch
   uint32_t* scan_tmp;        // block sums for the scans
   uint32_t* bbox_tmp;        // per target, then per source: 8 words of bounding-box partials

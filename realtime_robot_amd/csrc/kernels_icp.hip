@@ -37,7 +37,6 @@
 namespace rtr {
 
 constexpr uint32_t kFinishedBit = 1u << 30;
-constexpr int kMaxSpins = 1 << 22;
 
 // Synchronisation between workgroups.  Everything one workgroup hands to
 // another travels through two words: a problem's done count (an item's
@@ -62,6 +61,19 @@ __device__ __forceinline__ int load_relaxed(const int* p) {
 __device__ __forceinline__ void acquire_agent() { __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "agent"); }
 __device__ __forceinline__ void store_release(uint32_t* p, uint32_t v) {
   __hip_atomic_store(p, v, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_AGENT);
+}
+
+// A workgroup's wait for the next transform ends with the launch marked failed
+// when another wait did (the error flag, on its own cache line) or after
+// e.wait_ticks of the wall clock; both are looked at every 256 polls.  (A bound
+// on the number of polls shrank with the cost of a poll: with relaxed polls and
+// short sleeps 4M of them passed within the first iteration of 200k points
+// without seeds, and the call failed.)
+__device__ __forceinline__ bool wait_over(const DevEngine& e, int polls, uint64_t& since) {
+  if ((polls & 255) != 0) return false;
+  const uint64_t now = wall_clock64();
+  if (polls == 256) since = now;
+  return now - since > e.wait_ticks || load_relaxed((const uint32_t*)e.error) != 0u;
 }
 
 __device__ __forceinline__ GridView grid_of(const DevEngine& e, const TargetDesc& td) {
@@ -978,11 +990,11 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
           const uint32_t* word = (const uint32_t*)&e.st[p].gen;
           uint32_t wv = load_relaxed(word);
           int spins = 0;
-          // bounded wait with backoff; the error flag (on its own cache line)
-          // is polled every 256 rounds
+          uint64_t since = 0;
+          // bounded wait with backoff
           while (!(wv & kFinishedBit) && (int)wv < pass) {
             ++spins;
-            if (spins > kMaxSpins || ((spins & 255) == 0 && load_relaxed((const uint32_t*)e.error) != 0u)) {
+            if (wait_over(e, spins, since)) {
               atomicOr(e.error, 1);
               break;
             }
@@ -1159,9 +1171,10 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
           // bounded wait for this iteration's transform
           uint32_t wv = load_relaxed(word);
           int spins = 0;
+          uint64_t since = 0;
           while (!(wv & kFinishedBit) && (int)wv < pass) {
             ++spins;
-            if (spins > kMaxSpins || ((spins & 255) == 0 && load_relaxed((const uint32_t*)e.error) != 0u)) {
+            if (wait_over(e, spins, since)) {
               if (lane == 0) atomicOr(e.error, 1);
               break;
             }

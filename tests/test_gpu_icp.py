@@ -557,3 +557,26 @@ def test_correspondences_of_an_iteration_on_the_subsample():
         assert r["n_corr"] == got.sum() <= (len(src) + 3) // 4
         assert np.array_equal(idx[got], i_ref[got]) and np.array_equal(d2[got], d_ref[got])
         assert np.isinf(d2[~got]).all()
+
+
+def test_a_long_first_iteration_is_waited_for():
+    """200k points a metre beside a 200k-point target, no correspondence limit:
+    the first iteration, without seeds, takes longer than all others, and the
+    workgroups done with their share wait for it.  The wait's bound is there for
+    a launch that cannot end, not for this one; the result is the batch engine's."""
+    rng = np.random.default_rng(400000)
+    tgt, src = synth.sample_many([synth.CHAIR, synth.CHAIR], [200000, 200000], rng, 0.001)
+    src = synth.apply(synth.random_rigid(rng, 10.0, 0.05), src) + np.float32([0, 1, 0])
+    p = R.make_params(max_iterations=3)
+    icp = R.IterativeClosestPoint()
+    icp.set_params(p)
+    icp.setInputSource(src)
+    icp.setInputTarget(tgt)
+    icp.align()
+    reg = R.BatchRegistration()
+    reg.set_params(p)
+    reg.set_clouds([src], [tgt])
+    reg.set_problems([0], [0])
+    a, b = icp.getResult(), reg.align()[0]
+    assert a["iterations"] == b["iterations"] == 3 and a["n_corr"] == b["n_corr"] == len(src)
+    assert np.abs(a["T"] - b["T"]).max() < 1e-10 and abs(a["mse"] - b["mse"]) <= 1e-10 * b["mse"]
