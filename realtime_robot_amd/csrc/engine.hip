@@ -49,6 +49,10 @@ int Engine::init() {
   RTR_HIP(hipDeviceGetAttribute(&cu_count_, hipDeviceAttributeMultiprocessorCount, device_));
   RTR_HIP(hipDeviceGetAttribute(&wall_khz_, hipDeviceAttributeWallClockRate, device_));
   if (wall_khz_ <= 0) wall_khz_ = 100000;
+  for (int m = 0; m < 2; ++m)
+    one_most_[m] = std::min<uint32_t>(
+        (uint32_t)(cu_count_ * std::min(2, icp_one_blocks_per_cu(m ? RTR_MODE_POINT_TO_PLANE : RTR_MODE_POINT_TO_POINT))),
+        kOneItems);
   return RTR_OK;
 }
 
@@ -537,20 +541,21 @@ DevEngine Engine::dev_view() const {
 }
 
 // The one-registration kernel serves engines set up for single registrations
-// (TuneParams::single) while 256 queries' worth of workgroups on every CU reach
-// the whole source in a few rounds; beyond a million points the work, not the
-// chain of iterations, is what a launch waits for.
+// (TuneParams::single) while its items hold the source (k_icp_one has both
+// sides of the line).
 bool Engine::one_problem() const {
-  return tune_.single && probs_.size() == 1 && srcs_[probs_[0].src].n <= (1u << 20);
+  return tune_.single && probs_.size() == 1 && srcs_[probs_[0].src].n <= kOnePts * one_most();
 }
+
+// The workgroups of that kernel that are resident together: an item each.
+uint32_t Engine::one_most() const { return one_most_[prm_.mode == RTR_MODE_POINT_TO_PLANE ? 1 : 0]; }
 
 // Points per work item: as tuned, or for one problem 64 (one query per four
 // lanes of a workgroup) as long as the items fit the workgroups that can be
 // resident, else the next multiple of 64 that does.
 uint32_t Engine::item_points() const {
   if (!one_problem()) return (uint32_t)tune_.item_pts;
-  const uint32_t n = srcs_[probs_[0].src].n;
-  const uint32_t most = std::min<uint32_t>((uint32_t)(cu_count_ * std::min(2, icp_one_blocks_per_cu(prm_.mode))), kOneItems);
+  const uint32_t n = srcs_[probs_[0].src].n, most = one_most();
   return 64u * std::max(1u, (n + 64u * most - 1u) / (64u * most));
 }
 

@@ -122,6 +122,7 @@ class Engine {
   // list, and their size
   bool one_problem() const;
   uint32_t item_points() const;
+  uint32_t one_most() const;
 
   int device_;
   hipStream_t stream_ = nullptr;
@@ -137,6 +138,7 @@ class Engine {
   bool results_valid_ = false;  // states/grids hold a completed align of the current layout
   bool normals_valid_ = false;
   int cu_count_ = 0;
+  uint32_t one_most_[2] = {1, 1};  // most items of a one-problem launch, per mode
   int wall_khz_ = 0;  // rate of the device's wall clock
   rtr_params prm_;
   TuneParams tune_;

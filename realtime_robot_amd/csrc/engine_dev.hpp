@@ -89,7 +89,8 @@ void launch_source_sort(const DevEngine& e, int max_src_pts, hipStream_t s);
 void launch_icp(const DevEngine& e, int grid_blocks, hipStream_t s);
 int icp_blocks_per_cu(int mode, int use_tile, int variant);
 int icp_one_blocks_per_cu(int mode);
-constexpr uint32_t kOneItems = 1024;  // most work items of a one-problem launch
+constexpr uint32_t kOneItems = 1024;  // most work items of a one-problem launch ...
+constexpr uint32_t kOnePts = 256;     // ... and most points of one
 // correspondences / fitness / transformed output for problem set; T per
 // problem from `T` (n_prob*16 column-major, device) or from the state when null.
 void launch_correspondences(const DevEngine& e, int prob, const double* T, float r2f, int32_t* idx,

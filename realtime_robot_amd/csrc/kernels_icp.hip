@@ -1048,8 +1048,25 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
 // iteration to iteration.  A whole call on 2k x 10k points 1.70 -> 0.92 ms and
 // on 10k x 20k 2.23 -> 1.22 ms (38 -> 18 us an iteration, of which the sums and
 // the solve take 6); 30k x 366k points point-to-plane: the launch 1.0 -> 0.7 ms.
+//
+// A query without a seed in reach whose ball is wide needs the walk instead,
+// which takes the nearest rows first, and four lanes on one walk do one lane's
+// work.  While a workgroup holds 64 queries that costs nothing (its other lanes
+// would idle, and a wave then waits for the longest of 16 walks, not of 64).
+// Larger items (LISTED) put such queries on a list and walk it a lane each: the
+// first iteration of 100k x 100k points without a correspondence limit 1.96 ->
+// 1.15 ms, a metre off 82 -> 30 ms (the queue kernel: 1.03, 28).  Items have up
+// to kOnePts points, 131072 in a launch on 256 CUs; beyond, the queue kernel's
+// throughput wins: five iterations of 130k x 200k points take 0.90 ms here and
+// 1.06 there, of 200k x 200k 1.62 (items of 448) and 1.00.
 // ---------------------------------------------------------------------------
 constexpr int kOneQueries = kBlock / 4;  // queries a workgroup searches at a time
+
+// Items up to this size search small balls without a seed by four lanes (see
+// kQuadUnseeded), larger ones put these on the list too: five iterations of 50k
+// x 100k points (items of 128) 394 us, 459 by the list; of 100k x 100k (256) 653
+// us, 610 by the list.
+constexpr uint32_t kQuadUnseededItem = 128;
 
 template <int I>
 __device__ __forceinline__ uint32_t quad_bcast(uint32_t v) {
@@ -1117,11 +1134,13 @@ __device__ __forceinline__ void search_quad(const GridView& g, float qx, float q
   }
 }
 
-template <int MODE>
+template <int MODE, bool LISTED>
 __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
   constexpr int NS = MODE == RTR_MODE_POINT_TO_POINT ? SUM_P2P_COUNT : SUM_P2L_COUNT;
   __shared__ IcpShared<NS, WaveTileNone> sh;
   __shared__ uint16_t s_item[kOneItems];  // the items this workgroup keeps
+  __shared__ uint16_t s_walk[kWaves][LISTED ? kOnePts / kWaves : 1];  // an item's queries to walk, by wave
+  __shared__ uint32_t s_nwalk[kWaves];
   const int tid = threadIdx.x, lane = tid & 63, w = tid >> 6, sub = tid & 3;
   const Problem pr = scalar_copy(e.probs[0]);
   const SourceDesc sd = scalar_copy(e.srcs[pr.src]);
@@ -1130,6 +1149,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
   const float r2f = e.prm.r2f;
   const double ax = (double)td.anchor[0], ay = (double)td.anchor[1], az = (double)td.anchor[2];
   const uint32_t S = (uint32_t)e.item_pts;
+  const float unseeded = S <= kQuadUnseededItem ? kQuadUnseeded : 0.f;
   uint32_t* const seeds = e.nn_seed + pr.pt_off;
   const uint32_t* const word = (const uint32_t*)&e.st[0].gen;
   if (tid == 0) sh.n_search = 0u;
@@ -1202,6 +1222,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
       double acc[NS];
 #pragma unroll
       for (int k = 0; k < NS; ++k) acc[k] = 0.0;
+      uint32_t n_walk = 0u;  // this wave's queries left for the walk
       for (uint32_t base = first; base < end; base += kOneQueries) {
         float qx, qy, qz;
         int cx = 0, cy = 0, cz = 0;
@@ -1220,6 +1241,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
           D = e.cell_dist[td.cell_off + ((uint32_t)cz * g.dy + cy) * g.dx + cx];
           if (D >= td.skip_ring) act = false;
         }
+        bool walk = false;
         if (act) {
           n_search += sub == 0 ? 1u : 0u;
           const float bound = fminf(key_d2(key), r2f);
@@ -1227,9 +1249,10 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
           // nearest first, has to be small)
           const float side = sqrt_approx(bound) * g.inv_h;
           BallRows box;
-          if (side < (key != kNoKey ? 400.f : kQuadUnseeded) && ball_rows(g, qy, qz, bound * 1.000004f, box)) {
+          walk = !(side < (key != kNoKey ? 400.f : unseeded) && ball_rows(g, qy, qz, bound * 1.000004f, box));
+          if (!walk) {
             search_quad(g, qx, qy, qz, r2f, sub, box, key, where);
-          } else {
+          } else if (!LISTED) {
             GlobalVis<8> vis;
             vis.init(g, qx, qy, qz);
             vis.key = key;
@@ -1238,7 +1261,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
             key = vis.key;
             where = vis.where & 0x7fffffffu;
           }
-          if (sub == 0) {
+          if (sub == 0 && !(walk && LISTED)) {
             if (key != kNoKey && where != s0) seeds[j] = where;
             if (key_d2(key) <= r2f) {
               const float4 c = where == s0 ? t0 : g.pts[where];
@@ -1246,9 +1269,39 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
             }
           }
         }
+        if (LISTED) {
+          const bool put = walk && sub == 0;
+          const uint64_t bal = __ballot(put);
+          if (put) s_walk[w][n_walk + (uint32_t)__popcll(bal & ((1ull << lane) - 1ull))] = (uint16_t)(j - first);
+          n_walk += (uint32_t)__popcll(bal);
+        }
         if (base + kOneQueries < end) {
           j += kOneQueries;
           fetch(j);
+        }
+      }
+      if (LISTED) {
+        // the walks, a lane each (the lists in wave order, so that the sums are
+        // the same in every run)
+        if (lane == 0) s_nwalk[w] = n_walk;
+        __syncthreads();
+        const uint32_t w0 = s_nwalk[0], w1 = w0 + s_nwalk[1], w2 = w1 + s_nwalk[2], total = w2 + s_nwalk[3];
+        for (uint32_t t = (uint32_t)tid; t < total; t += kBlock) {
+          const int l = t < w0 ? 0 : (t < w1 ? 1 : (t < w2 ? 2 : 3));
+          const uint32_t jj = first + s_walk[l][t - (l == 0 ? 0u : (l == 1 ? w0 : (l == 2 ? w1 : w2)))];
+          float qx, qy, qz;
+          int cx, cy, cz;
+          apply_f32(m, e.sx[sd.off + jj], e.sy[sd.off + jj], e.sz[sd.off + jj], qx, qy, qz);
+          query_cell(g, qx, qy, qz, cx, cy, cz);
+          const uint32_t seed = pass > 0 ? seeds[jj] : ~0u;
+          GlobalVis<8> vis;
+          vis.init(g, qx, qy, qz);
+          if (seed - g.pt_lo < g.n_pts) vis.seed(seed);
+          const int D = e.cell_dist ? (int)e.cell_dist[td.cell_off + ((uint32_t)cz * g.dy + cy) * g.dx + cx] : 0;
+          search_global(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
+          const uint32_t at = vis.where & 0x7fffffffu;
+          if (vis.key != kNoKey && at != seed) seeds[jj] = at;
+          if (key_d2(vis.key) <= r2f) add_pair<MODE>(e, qx, qy, qz, g.pts[at], at, key_d2(vis.key), ax, ay, az, acc);
         }
       }
       wave_totals<NS>(acc, sh, w, lane, false);
@@ -1293,12 +1346,17 @@ int icp_blocks_per_cu(int mode, int use_tile, int variant) {
                   : blocks_per_cu_of<RTR_MODE_POINT_TO_POINT, false, 4, 3>();
 }
 
-int icp_one_blocks_per_cu(int mode) {
+template <int MODE, bool LISTED>
+static int one_blocks_per_cu_of() {
   int nb = 0;
-  const hipError_t rc = mode == RTR_MODE_POINT_TO_PLANE
-                            ? hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_icp_one<RTR_MODE_POINT_TO_PLANE>, kBlock, 0)
-                            : hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_icp_one<RTR_MODE_POINT_TO_POINT>, kBlock, 0);
+  const hipError_t rc = hipOccupancyMaxActiveBlocksPerMultiprocessor(&nb, k_icp_one<MODE, LISTED>, kBlock, 0);
   return rc != hipSuccess || nb < 1 ? 1 : nb;
+}
+
+int icp_one_blocks_per_cu(int mode) {
+  return mode == RTR_MODE_POINT_TO_PLANE
+             ? std::min(one_blocks_per_cu_of<RTR_MODE_POINT_TO_PLANE, false>(), one_blocks_per_cu_of<RTR_MODE_POINT_TO_PLANE, true>())
+             : std::min(one_blocks_per_cu_of<RTR_MODE_POINT_TO_POINT, false>(), one_blocks_per_cu_of<RTR_MODE_POINT_TO_POINT, true>());
 }
 
 void launch_icp(const DevEngine& e, int grid_blocks, hipStream_t s) {
@@ -1307,10 +1365,11 @@ void launch_icp(const DevEngine& e, int grid_blocks, hipStream_t s) {
   hipLaunchKernelGGL(k_icp_init, dim3(init_blocks), dim3(kBlock), 0, s, e);
   const dim3 g(grid_blocks), b(kBlock);
   if (e.one) {
-    if (e.prm.mode == RTR_MODE_POINT_TO_PLANE)
-      hipLaunchKernelGGL(k_icp_one<RTR_MODE_POINT_TO_PLANE>, g, b, 0, s, e);
-    else
-      hipLaunchKernelGGL(k_icp_one<RTR_MODE_POINT_TO_POINT>, g, b, 0, s, e);
+    const bool listed = e.item_pts > kOneQueries;
+    auto* kernel = e.prm.mode == RTR_MODE_POINT_TO_PLANE
+                       ? (listed ? k_icp_one<RTR_MODE_POINT_TO_PLANE, true> : k_icp_one<RTR_MODE_POINT_TO_PLANE, false>)
+                       : (listed ? k_icp_one<RTR_MODE_POINT_TO_POINT, true> : k_icp_one<RTR_MODE_POINT_TO_POINT, false>);
+    hipLaunchKernelGGL(kernel, g, b, 0, s, e);
     return;
   }
   if (e.prm.mode == RTR_MODE_POINT_TO_PLANE) {

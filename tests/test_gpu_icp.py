@@ -580,3 +580,73 @@ def test_a_long_first_iteration_is_waited_for():
     a, b = icp.getResult(), reg.align()[0]
     assert a["iterations"] == b["iterations"] == 3 and a["n_corr"] == b["n_corr"] == len(src)
     assert np.abs(a["T"] - b["T"]).max() < 1e-10 and abs(a["mse"] - b["mse"]) <= 1e-10 * b["mse"]
+
+
+@pytest.mark.parametrize("ns", [32769, 50000, 65537, 98000, 131072, 131073])
+@pytest.mark.parametrize("kw", [dict(), dict(max_correspondence_distance=0.05),
+                                dict(max_correspondence_distance=0.3, cell_size=0.02),
+                                dict(max_correspondence_distance=0.05, coarse_stride=3, coarse_iterations=2),
+                                dict(max_correspondence_distance=0.1, mode=1)])
+def test_one_registration_kernel_on_larger_items(ns, kw):
+    """Items of 128 to 256 points, and the first size past them, where the queue
+    takes over: queries without a seed in reach are left to a lane each there.
+    Every second point starts out of reach and every seventh is not finite, so
+    that seeds are missing in every iteration; against the batch engine as in
+    the test of the smaller sizes."""
+    rng = np.random.default_rng(ns)
+    tgt, src = synth.sample_many([synth.CHAIR, synth.CHAIR], [20000, ns], rng, 0.002)
+    src = synth.apply(synth.random_rigid(rng, 8.0, 0.03), src)
+    src[1::2] += np.float32([0.0, 0.2, 0.1])
+    src[3::7] = np.nan
+    p = R.make_params(**dict(dict(max_iterations=5), **kw))
+    icp = R.IterativeClosestPoint()
+    icp.set_params(p)
+    icp.setInputSource(src)
+    icp.setInputTarget(tgt)
+    reg = R.BatchRegistration()
+    reg.set_params(p)
+    reg.set_clouds([src], [tgt])
+    reg.set_problems([0], [0])
+    if kw.get("mode"):
+        icp.computeTargetNormals(10, (0.0, 0.0, 3.0))
+        reg.compute_target_normals(10, (0.0, 0.0, 3.0))
+    b = reg.align()[0]
+    first = None
+    for rep in range(2):
+        icp.align()
+        a = icp.getResult()
+        for k in ("iterations", "state", "n_corr", "coarse_iterations"):
+            assert a[k] == b[k], k
+        assert np.abs(a["T"] - b["T"]).max() < 1e-10 and abs(a["mse"] - b["mse"]) <= 1e-10 * b["mse"]
+        assert icp.getTiming()["queries_searched"] == reg.timing()["queries_searched"]
+        assert first is None or np.array_equal(first, a["T"])   # sums in a fixed order
+        first = a["T"].copy()
+
+
+def test_one_registration_kernel_keeps_its_lanes_busy():
+    """Without seeds four lanes on one query's walk do a quarter of the work: the
+    launch, on 100k points a metre off, takes no longer than the queue kernel on
+    the same items, give or take half (28 against 29 ms; 82 with idle lanes)."""
+    rng = np.random.default_rng(200000)
+    tgt, src = synth.sample_many([synth.CHAIR, synth.CHAIR], [100000, 100000], rng, 0.001)
+    src = synth.apply(synth.random_rigid(rng, 10.0, 0.05), src) + np.float32([1, 0, 0])
+    p = R.make_params(max_iterations=1)
+    icp = R.IterativeClosestPoint()
+    icp.set_params(p)
+    icp.set_profiling(True)
+    icp.setInputSource(src)
+    icp.setInputTarget(tgt)
+    reg = R.BatchRegistration()
+    reg.set_tuning(item_pts=256, blocks_per_cu=1)
+    reg.set_params(p)
+    reg.set_profiling(True)
+    reg.set_clouds([src], [tgt])
+    reg.set_problems([0], [0])
+    one, queue = [], []
+    for rep in range(4):
+        icp.align()
+        reg.align()
+        one.append(icp.getTiming()["ms_icp"])
+        queue.append(reg.timing()["ms_icp"])
+    print(min(one), min(queue))
+    assert min(one) < 1.5 * min(queue)
