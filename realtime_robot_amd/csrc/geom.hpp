@@ -420,6 +420,23 @@ RTR_HD void walk_ball(const GridView& g, float qx, float qy, float qz, int cx, i
   }
 }
 
+// A squared distance within which a query without a seed has a target point, from
+// the distance field's value D of its cell: some cell at Chebyshev distance D
+// holds one, and the farthest corner of the (2D + 1)^3 block of cells, less
+// exact by the margin, is the farthest it can be.  Unbounded where the field is
+// at its cap (see dist_caps).  Without it the ball of r_max is all that an
+// unseeded walk has to go by: its first rows are then read r_max to each side.
+constexpr int kDistCap = 14;
+RTR_HD float dist_bound2(const GridView& g, float qx, float qy, float qz, int cx, int cy, int cz, int D) {
+  if (D > kDistCap) return 3.4e38f;
+  auto far = [&](float q, float o, int c) {
+    const float a = q - (o + (float)(c - D) * g.h), b = (o + (float)(c + D + 1) * g.h) - q;
+    return (a > b ? a : b) + g.margin;
+  };
+  const float x = far(qx, g.ox, cx), y = far(qy, g.oy, cy), z = far(qz, g.oz, cz);
+  return (x * x + y * y + z * z) * 1.000004f;
+}
+
 // The rows (y, z) of cells that the ball of squared radius B about a query can
 // meet, as one list in which lanes take a row each: all rows of a box, found as
 // walk_ball finds a row's cells.  False when a side has more than kBallSide
@@ -484,18 +501,18 @@ RTR_HD void dist_caps(float r_max, float h, float margin, int* skip_ring, int* d
   const double rr = ((double)r_max + (double)margin) / (double)h;
   if (!(rr < 12.0)) {
     *skip_ring = 255;
-    *dt_cap = 14;
+    *dt_cap = kDistCap;
   } else {
     *skip_ring = (int)floor(rr) + 2;
-    *dt_cap = *skip_ring < 14 ? *skip_ring : 14;
+    *dt_cap = *skip_ring < kDistCap ? *skip_ring : kDistCap;
   }
 }
 
 // The ICP search of one query (k_icp's, on any visitor): the cell's distance D
 // (a lower bound on the Chebyshev distance to the nearest occupied cell) is
 // consulted first, D >= skip_ring means no point within r_max.  With a finite
-// bound, from the visitor's seed or from r2f, one walk over the ball's rows;
-// else rings, from shell D when D >= 2 shows the 3x3x3 block empty.
+// bound, from the visitor's seed, from r2f or from D, one walk over the ball's
+// rows; else rings, from shell D when D >= 2 shows the 3x3x3 block empty.
 template <class V>
 RTR_HD void ring_walk_dt(const GridView& g, const uint8_t* dist, int skip_ring, float qx, float qy,
                          float qz, float r2f, V& vis) {
@@ -503,8 +520,13 @@ RTR_HD void ring_walk_dt(const GridView& g, const uint8_t* dist, int skip_ring, 
   if (!query_cell(g, qx, qy, qz, cx, cy, cz)) return;
   const int D = dist[((uint32_t)cz * g.dy + cy) * g.dx + cx];
   if (D >= skip_ring) return;
-  if ((vis.bound() < r2f ? vis.bound() : r2f) < 1.0e30f) {
-    walk_ball(g, qx, qy, qz, cx, cy, cz, D, r2f, vis);
+  float reach = r2f;
+  if (vis.bound() > 1.0e30f) {
+    const float b = dist_bound2(g, qx, qy, qz, cx, cy, cz, D);
+    reach = b < reach ? b : reach;
+  }
+  if ((vis.bound() < reach ? vis.bound() : reach) < 1.0e30f) {
+    walk_ball(g, qx, qy, qz, cx, cy, cz, D, reach, vis);
     return;
   }
   int k0 = 1;

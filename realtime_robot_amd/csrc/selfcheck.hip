@@ -19,9 +19,9 @@ namespace rtr {
 // k_icp_one's search of a seeded query, four rows at a time, one after the
 // other: false when its rows are more than it takes.  A row outside the grid or
 // a range outside the target sets *bad.
-static bool quad_search(const GridView& g, float r2f, NNCountVisitor& v, bool* bad) {
+static bool quad_search(const GridView& g, float reach, NNCountVisitor& v, bool* bad) {
   BallRows box;
-  float B = std::fmin(v.bound(), r2f) * 1.000004f;
+  float B = std::fmin(v.bound(), reach) * 1.000004f;
   if (!ball_rows(g, v.qy, v.qz, B, box)) return false;
   if (box.ny <= 0 || box.nz <= 0) return true;
   const int nrows = box.ny * box.nz;
@@ -42,7 +42,7 @@ static bool quad_search(const GridView& g, float r2f, NNCountVisitor& v, bool* b
       }
     }
     for (int u = 0; u < 4; ++u) v.scan(b[u], e[u]);
-    B = std::fmin(v.bound(), r2f) * 1.000004f;
+    B = std::fmin(v.bound(), reach) * 1.000004f;
   }
   return true;
 }
@@ -174,7 +174,15 @@ int rtr_selfcheck_nn_stats(const float* tgt, size_t nt, const float* q, size_t n
       // k_icp_one's search from the same start has to find the same point
       NNCountVisitor one = v, walk = v;
       bool bad = false;
-      if (((i & 1) || std::sqrt(r2f) * g.inv_h < kQuadUnseeded) && quad_search(g, r2f, one, &bad)) {
+      float reach = r2f;
+      if (!(i & 1)) {
+        const int D = da[((size_t)cz * g.dy + cy) * g.dx + cx];
+        if (D >= skip_ring)
+          reach = -1.f;
+        else
+          reach = std::fmin(r2f, dist_bound2(g, v.qx, v.qy, v.qz, cx, cy, cz, D));
+      }
+      if (reach >= 0.f && ((i & 1) || std::sqrt(reach) * g.inv_h < kQuadUnseeded) && quad_search(g, reach, one, &bad)) {
         ring_walk_dt(g, da.data(), skip_ring, v.qx, v.qy, v.qz, r2f, walk);
         const bool found = key_d2(walk.best.key) <= r2f;
         if (bad || (found ? one.best.key != walk.best.key : key_d2(one.best.key) <= r2f)) {

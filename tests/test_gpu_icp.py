@@ -650,3 +650,31 @@ def test_one_registration_kernel_keeps_its_lanes_busy():
         queue.append(reg.timing()["ms_icp"])
     print(min(one), min(queue))
     assert min(one) < 1.5 * min(queue)
+
+
+@pytest.mark.parametrize("n,cell", [(10000, 0.02), (10000, 0.04), (60000, 0.04)])
+def test_a_wide_limit_costs_a_first_iteration_nothing(n, cell):
+    """Without a seed the walk's reach is what the distance field allows, not the
+    correspondence limit: one iteration with a limit of 30 cells takes about as
+    long as with one of 3 (give or take half; up to 1.9 times as long when the
+    walk began with the limit's ball), and finds what brute force finds."""
+    rng = np.random.default_rng(n)
+    tgt, src = synth.sample_many([synth.CHAIR, synth.CHAIR], [n, n], rng, 0.001)
+    src = synth.apply(synth.random_rigid(rng, 10.0, 0.05), src)
+    ms = []
+    for cells in (3, 30):
+        b = R.BatchRegistration()
+        b.set_params(R.make_params(max_iterations=1, max_correspondence_distance=cells * cell, cell_size=cell,
+                                   cells_per_point=30.0))
+        b.set_profiling(True)
+        b.set_clouds([src], [tgt])
+        b.set_problems([0] * 8, [0] * 8)
+        for rep in range(5):
+            b.align()
+            ms.append((cells, b.timing()["ms_icp"]))
+        idx, d2 = b.last_correspondences(7)
+        i_ref, d_ref = oracle.nn_brute(src, tgt, cells * cell)
+        assert np.array_equal(idx, i_ref) and np.array_equal(d2, d_ref)
+    near, wide = (min(t for c, t in ms if c == cells) for cells in (3, 30))
+    print(near, wide)
+    assert wide < 1.5 * near
