@@ -51,56 +51,130 @@ __global__ void k_tdf_mark_points(const float* xyz, size_t n, float ox, float oy
 }
 
 // One pass along axis A (0 = x, 1 = y, 2 = z): out(a) = min(cap, min_t
-// (a - t)^2 + in(t)) over the line through the voxel, one voxel per lane.  The
-// offsets go outward and stop at the first r with r^2 >= the best so far: no
-// farther term can be smaller (its rounded sum is at least r^2), so the result
-// is that of the whole line, bit for bit.  Capping every pass, not the last
-// alone, changes nothing either (a term with in >= cap is >= cap) and bounds
-// the offsets by sqrt(cap) where a line holds nothing.  Lanes run along x, so
-// every load of the three passes is one contiguous segment per wave; four
-// offsets to each side are in flight at once.
+// (a - t)^2 + in(t)) over the line through the voxel.  The offsets go outward
+// and stop at the first r with r^2 >= the best so far: no farther term can be
+// smaller (its rounded sum is at least r^2), so the result is that of the whole
+// line, bit for bit.  Capping every pass, not the last alone, changes nothing
+// either (a term with in >= cap is >= cap) and bounds the offsets by sqrt(cap)
+// where a line holds nothing.
 //
-// Staging whole lines in LDS and taking all len terms (len^2 per line) was
-// VALU-bound: 405, 411 and 231 us for 250 x 250 x 125 at cap 900; 95, 94 and 124 now,
-// bound by the latency of the loads (the field is 31 MB: L2 and MALL).
-template <int A>
-__global__ __launch_bounds__(256) void k_tdf_pass(const float* in, float* out, uint32_t n, int dx, int dy, int dz,
+// A lane takes R neighbouring voxels of its line, so that a value read serves
+// them all, with U offsets to each side in flight.  Lanes run along x in the y
+// and z passes, and every load is then one contiguous segment per wave.
+//
+// Large fields (R = 4, U = 4) are bound by their loads and addresses, most of
+// all where nothing stops the offsets (a large cap, few occupied voxels): with
+// one voxel a lane such passes took longer than all terms of the line from LDS
+// had.  250 x 250 x 125, the three passes: one occupied voxel and cap 10^9, from
+// LDS 1057 us, one voxel a lane 1641, now 851; cap 900, 1058, 369, 176; 300k
+// occupied, cap 900, 1058, 155, 93.  Small fields leave the chip idle and are a
+// chain of load latencies: R = 1 for more lanes, and more offsets at once.
+// 30^3, five launches: from LDS 15.0-17.1 us, U = 4 17.3-20.3, U = 16 15.0-16.9;
+// 50^3 27, 24 (U = 4), 23 (U = 8), 29 (R = 4); 64^3, cap 10^9: 37, 33, 35 (U = 8),
+// 32 (R = 4).
+template <int A, int R, int U>
+__global__ __launch_bounds__(256) void k_tdf_pass(const float* in, float* out, uint32_t n_runs, int dx, int dy, int dz,
                                                   float cap) {
-  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n; i += gridDim.x * 256u) {
-    const uint32_t q = i / (uint32_t)dx;
-    const int pos = A == 0 ? (int)(i - q * (uint32_t)dx) : (A == 1 ? (int)(q % (uint32_t)dy) : (int)(q / (uint32_t)dy));
-    const int len = A == 0 ? dx : (A == 1 ? dy : dz);
-    const ptrdiff_t stride = A == 0 ? 1 : (A == 1 ? dx : (ptrdiff_t)dx * dy);
-    const float* p = in + i;
-    const int lo = pos, hi = len - 1 - pos, far = lo > hi ? lo : hi;  // offsets inside the line
-    float best = fminf(*p, cap);
-    for (int r = 1; r <= far && (float)r * (float)r < best; r += 4) {
-      float a[4], b[4];
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        a[u] = p[-(ptrdiff_t)min(r + u, lo) * stride];
-        b[u] = p[(ptrdiff_t)min(r + u, hi) * stride];
-      }
-#pragma unroll
-      for (int u = 0; u < 4; ++u) {
-        // (an offset past the line's end repeats the end voxel's value at a
-        // larger distance than its own: never below the term it stands for)
-        const float d = (float)(r + u) * (float)(r + u);
-        best = fminf(best, fminf(d + a[u], d + b[u]));
+  const int len = A == 0 ? dx : (A == 1 ? dy : dz);
+  const ptrdiff_t stride = A == 0 ? 1 : (A == 1 ? dx : (ptrdiff_t)dx * dy);
+  const uint32_t per_line = (uint32_t)(len + R - 1) / R;
+  for (uint32_t i = blockIdx.x * 256u + threadIdx.x; i < n_runs; i += gridDim.x * 256u) {
+    // the run's first voxel: runs along x, y or z in place of voxels
+    int pos;
+    size_t at;
+    if (A == 0) {
+      const uint32_t line = i / per_line;
+      pos = R * (int)(i - line * per_line);
+      at = (size_t)line * dx + pos;
+    } else {
+      const uint32_t q = i / (uint32_t)dx, x = i - q * (uint32_t)dx;
+      if (A == 1) {
+        const uint32_t z = q / per_line;
+        pos = R * (int)(q - z * per_line);
+        at = x + (size_t)dx * ((size_t)z * dy + pos);
+      } else {
+        const uint32_t g = q / (uint32_t)dy;
+        pos = R * (int)g;
+        at = x + (size_t)dx * ((q - g * (uint32_t)dy) + (size_t)pos * dy);
       }
     }
-    out[i] = best;
+    const int m = min(R, len - pos);  // voxels of the run: fewer at the line's end
+    const float* const p = in + at;
+    const float* const e = p + (m - 1) * stride;
+    float v[R], best[R];
+#pragma unroll
+    for (int k = 0; k < R; ++k) v[k] = p[min(k, m - 1) * stride];
+#pragma unroll
+    for (int k = 0; k < R; ++k) {
+      best[k] = fminf(v[k], cap);
+#pragma unroll
+      for (int j = 0; j < R; ++j)
+        if (j != k) best[k] = fminf(best[k], (float)((k - j) * (k - j)) + v[j]);
+    }
+    // (an offset past the line's end, here and below, repeats the end voxel's
+    // value at a distance no shorter than its own: never below the term it
+    // stands for)
+    const int lo = pos, hi = len - pos - m, both = min(lo, hi), far = max(lo, hi);
+    const float *l = p - stride, *h = e + stride;
+    auto largest = [&] {
+      float x = best[0];
+#pragma unroll
+      for (int k = 1; k < R; ++k) x = fmaxf(x, best[k]);
+      return x;
+    };
+    float lim = largest();
+    for (int r = 1; r <= far && (float)r * (float)r < lim; r += U, l -= U * stride, h += U * stride) {
+      float a[U], b[U];
+      if (r + U - 1 <= both) {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          a[u] = l[-u * stride];
+          b[u] = h[u * stride];
+        }
+      } else {
+#pragma unroll
+        for (int u = 0; u < U; ++u) {
+          a[u] = p[-min(r + u, lo) * stride];
+          b[u] = e[min(r + u, hi) * stride];
+        }
+      }
+      float d[U + R - 1];
+#pragma unroll
+      for (int j = 0; j < U + R - 1; ++j) d[j] = (float)(r + j) * (float)(r + j);
+#pragma unroll
+      for (int u = 0; u < U; ++u)
+#pragma unroll
+        for (int k = 0; k < R; ++k) best[k] = fminf(best[k], fminf(d[u + k] + a[u], d[u + R - 1 - k] + b[u]));
+      lim = largest();
+    }
+#pragma unroll
+    for (int k = 0; k < R; ++k)
+      if (k < m) out[at + k * stride] = best[k];
   }
 }
 
 // The three passes over n = dx dy dz <= 2^31 voxels, from a through b back to
 // a, and into out.
+template <int R, int U>
+static void tdf_passes_of(float* a, float* b, float* out, const int dims[3], float cap, hipStream_t s) {
+  const dim3 t(256);
+  auto runs = [&](int axis) {
+    return (uint32_t)((size_t)dims[0] * dims[1] * dims[2] / dims[axis] * ((dims[axis] + R - 1) / R));
+  };
+  auto grid = [](uint32_t n) { return dim3(std::min((n + 255u) / 256u, 1u << 20)); };
+  hipLaunchKernelGGL((k_tdf_pass<0, R, U>), grid(runs(0)), t, 0, s, a, b, runs(0), dims[0], dims[1], dims[2], cap);
+  hipLaunchKernelGGL((k_tdf_pass<1, R, U>), grid(runs(1)), t, 0, s, b, a, runs(1), dims[0], dims[1], dims[2], cap);
+  hipLaunchKernelGGL((k_tdf_pass<2, R, U>), grid(runs(2)), t, 0, s, a, out, runs(2), dims[0], dims[1], dims[2], cap);
+}
+
 static void tdf_passes(float* a, float* b, float* out, const int dims[3], float cap, hipStream_t s) {
-  const uint32_t n = (uint32_t)((size_t)dims[0] * dims[1] * dims[2]);
-  const dim3 g(std::min((n + 255u) / 256u, 1u << 20)), t(256);
-  hipLaunchKernelGGL(k_tdf_pass<0>, g, t, 0, s, a, b, n, dims[0], dims[1], dims[2], cap);
-  hipLaunchKernelGGL(k_tdf_pass<1>, g, t, 0, s, b, a, n, dims[0], dims[1], dims[2], cap);
-  hipLaunchKernelGGL(k_tdf_pass<2>, g, t, 0, s, a, out, n, dims[0], dims[1], dims[2], cap);
+  const size_t n = (size_t)dims[0] * dims[1] * dims[2];
+  if (n <= (size_t)1 << 16)
+    tdf_passes_of<1, 16>(a, b, out, dims, cap, s);
+  else if (n <= (size_t)1 << 17)
+    tdf_passes_of<1, 8>(a, b, out, dims, cap, s);
+  else
+    tdf_passes_of<4, 4>(a, b, out, dims, cap, s);
 }
 
 // Fills, marks, transforms and reads back; mem holds two fields and the input.

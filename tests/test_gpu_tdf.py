@@ -47,3 +47,18 @@ def test_outward_passes_match_brute_force(dims, cap):
     face = np.stack([np.zeros(8, np.int32), *(rng.integers(0, d[a], 8) for a in (1, 2))], 1).astype(np.int32)
     for occ in (one, face, np.zeros((0, 3), np.int32)):
         assert np.array_equal(R.tdf(occ, dims, cap), oracle.tdf(occ, dims, cap))
+
+
+@pytest.mark.parametrize("dims", [(41, 43, 45), (300, 17, 16), (4096, 6, 3), (70, 61, 33), (4, 9, 4000), (4096, 33, 1),
+                                  (1, 4096, 33), (129, 130, 11)])
+@pytest.mark.parametrize("cap", [900.0, 1.0e9])
+def test_passes_by_field_size_match_brute_force(dims, cap):
+    """The passes change with the field's size (one voxel a lane and eight or
+    sixteen offsets at once, or runs of four voxels): lines that end in every part
+    of a run, shorter than one, and longer than the offsets ever go."""
+    rng = np.random.default_rng(sum(dims))
+    d = np.array(dims)
+    few = (rng.random((3, 3)) * d).astype(np.int32)
+    many = (rng.random((2000, 3)) * d).astype(np.int32)
+    for occ in (few, many):
+        assert np.array_equal(R.tdf(occ, dims, cap), oracle.tdf(occ, dims, cap))
