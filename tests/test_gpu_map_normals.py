@@ -1,5 +1,7 @@
 """GPU parity: k-NN PCA normals, point-to-plane ICP, voxel-hash fusion and
 voxel-grid downsampling against the CPU oracle."""
+import ctypes as C
+
 import numpy as np
 import pytest
 
@@ -7,6 +9,7 @@ import oracle
 import realtime_robot_amd as R
 from helpers import golden, rot_err, trans_err
 from pcd_np import read_xyz
+from realtime_robot_amd import _lib as L
 from realtime_robot_amd import synth
 
 pytestmark = pytest.mark.gpu
@@ -310,3 +313,34 @@ def test_map_readout_order_and_reuse(shape, n):
     assert np.allclose(sums, mean * counts[:, None], rtol=2e-7, atol=2e-6 * counts.max())
     d = R.voxel_downsample(p, float(h))
     assert d.shape == mean.shape and np.all(np.abs(d - mean) <= tol)
+
+
+@pytest.mark.parametrize("n", [1, 2047, 2048, 2049, 5000])
+def test_map_readout_around_its_sizes(n):
+    """Few voxels are sorted on the host, more through the bit map: the same
+    order on both sides of the line, the number of voxels with an error when the
+    buffer is short of it, and again after a clear, also of an overfull map."""
+    rng = np.random.default_rng(n)
+    cell = rng.permutation(40 ** 3)[:n]
+    k = np.stack([cell % 40, cell // 40 % 40, cell // 1600], 1) - 20
+    p = ((k + 0.25) * 0.125).astype(np.float32)
+    key = np.sort((k[:, 0] + (1 << 20)) | ((k[:, 1] + (1 << 20)) << 21) | ((k[:, 2] + (1 << 20)) << 42))
+    m = R.VoxelMap(0.125, capacity=n)
+    for rep in range(2):
+        m.integrate(p)
+        gk, gx, gc = m.extract()
+        assert np.array_equal(gk, key) and (gc == 1).all()
+        order = np.lexsort((k[:, 0], k[:, 1], k[:, 2]))
+        assert np.array_equal(gx, p[order])     # a voxel's one point, exact in these units
+        size = C.c_size_t()
+        keys = np.empty(n, np.int64)
+        rc = L.lib.rtr_map_extract(m._h, L.ptr(keys), None, None, n - 1, C.byref(size), 1)
+        assert rc == 4 and size.value == n      # capacity
+        with pytest.raises(R.RtrError):
+            m.integrate(p + np.float32(16.0))   # as many again: more than the capacity
+        # (what fits the table beyond the capacity is kept, what its probes do not place is dropped)
+        assert n < m.size() <= 2 * n and m.size() + m.dropped() == 2 * n
+        gk, _, gc = m.extract()
+        assert len(gk) == m.size() and (np.diff(gk) > 0).all() and gc.sum() == m.size()
+        m.clear()
+        assert m.size() == 0 and len(m.extract()[0]) == 0
