@@ -1654,6 +1654,15 @@ __global__ __launch_bounds__(kNrmBlock) __attribute__((amdgpu_waves_per_eu(3))) 
   const GridView g = grid_of(e, td);
   const uint32_t base = e.cell_start[td.cell_off];
   const float* const raw = e.tgt_raw + 3 * (size_t)td.raw_off;
+  if (td.n_valid < td.n) {
+    // non-finite points are in no cell, and have no normal
+    for (uint32_t i = blockIdx.x * blockDim.x + threadIdx.x; i < td.n; i += gridDim.x * blockDim.x) {
+      const float* p = raw + 3 * (size_t)i;
+      if (isfinite(p[0]) && isfinite(p[1]) && isfinite(p[2])) continue;
+      float* o = nrm_raw + 3 * ((size_t)td.raw_off + i);
+      o[0] = o[1] = o[2] = __builtin_nanf("");
+    }
+  }
   for (uint32_t j0 = blockIdx.x * blockDim.x; j0 < td.n_valid; j0 += gridDim.x * blockDim.x) {
     const uint32_t j = j0 + threadIdx.x;
     if (j >= td.n_valid) continue;

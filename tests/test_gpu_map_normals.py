@@ -56,6 +56,47 @@ def test_normals_for_every_list_form(k, n):
     assert np.abs(icp.getFinalTransformation() - np.eye(4)).max() < 1e-6
 
 
+@pytest.mark.parametrize("k", [7, 20])
+def test_batch_normals_among_targets_with_nonfinite_points(k):
+    """Several targets, some with non-finite points, whose slots in the sorted
+    arrays then lie before their raw offsets: an align on the grids the normals
+    were computed on equals one on grids built from scratch with the normals
+    that each target gets by itself, bit for bit.  A non-finite point has no
+    normal, whatever was set before."""
+    rng = np.random.default_rng(k)
+    tgts, srcs, nrm = [], [], []
+    for j in range(5):
+        t = synth.sample_many([synth.CHAIR], [900 + 200 * j], rng, 0.002)[0]
+        srcs.append(synth.apply(synth.random_rigid(rng, 4.0, 0.02), t[::2]))
+        if j % 2 == 0:
+            t[rng.integers(0, len(t), 40), rng.integers(0, 3, 40)] = np.float32([np.nan, np.inf, -np.inf, np.nan] * 10)
+        tgts.append(t)
+        icp = R.IterativeClosestPointWithNormals()
+        icp.setInputSource(srcs[-1])
+        icp.setInputTarget(t)
+        icp.setTargetNormals(np.ones_like(t))
+        icp.computeTargetNormals(k, (0.0, 0.0, 3.0))
+        nrm.append(icp.getTargetNormals())
+        bad = ~np.isfinite(t).all(1)
+        assert np.isnan(nrm[-1][bad]).all() and np.isfinite(nrm[-1][~bad]).all()
+        assert np.abs(nrm[-1][~bad] - oracle.normals(t[~bad], k, vp=(0.0, 0.0, 3.0))[0]).max() < 1e-5
+    out = []
+    for own in (False, True):
+        b = R.BatchRegistration()
+        b.set_params(R.make_params(max_iterations=8, max_correspondence_distance=0.1, mode=1))
+        b.set_rebuild(own)
+        b.set_clouds(srcs, tgts)
+        if own:
+            b.set_target_normals(nrm)
+        b.set_problems(np.arange(5), np.arange(5))
+        if not own:
+            b.compute_target_normals(k, (0.0, 0.0, 3.0))
+        out.append(b.align())
+    for p in range(5):
+        assert out[0][p]["n_corr"] == out[1][p]["n_corr"] > 100
+        assert np.array_equal(out[0][p]["T"], out[1][p]["T"]) and out[0][p]["mse"] == out[1][p]["mse"], p
+
+
 def test_point_to_plane_matches_oracle():
     src, tgt, T_gt = synth.config1_pair(1)
     nrm, _ = oracle.normals(tgt, 20, vp=(0.0, 0.0, 2.0))
