@@ -37,11 +37,16 @@ def test_normals_for_every_list_form(k, n):
     Both sum the same k points in ascending (distance, index) order in FP64,
     so away from ties of the eigenvalues only the final float32 rounding is
     left: 1e-5 covers it with a relative eigenvalue gap down to 1e-10.  Fewer
-    than three points give NaN.  The align that follows uses the same grid."""
+    than three points give NaN.  The align that follows uses the grid that the
+    normals were computed on, with the normals the kernel left in cell order:
+    the same result, bit for bit, as on a handle that is given these normals and
+    builds its grid from scratch, and the oracle's, which it would not be with
+    every normal at its neighbour's place."""
     rng = np.random.default_rng(100 * k + n)
     tgt = rng.uniform(-1, 1, (n, 3)).astype(np.float32) * np.float32([1.0, 0.7, 0.02])
+    src = synth.apply(synth.random_rigid(np.random.default_rng(n), 2.0, 0.02), tgt)
     icp = R.IterativeClosestPointWithNormals()
-    icp.setInputSource(tgt)
+    icp.setInputSource(src)
     icp.setInputTarget(tgt)
     icp.computeTargetNormals(k, (0.0, 0.0, 2.0))
     got = icp.getTargetNormals()
@@ -50,10 +55,23 @@ def test_normals_for_every_list_form(k, n):
         assert np.isnan(got).all()
         return
     assert np.abs(got - ref).max() < 1e-5
-    icp.setMaxCorrespondenceDistance(0.5)
-    icp.setMaximumIterations(3)
-    icp.align()
-    assert np.abs(icp.getFinalTransformation() - np.eye(4)).max() < 1e-6
+    other = R.IterativeClosestPointWithNormals()
+    other.setInputSource(src)
+    other.setInputTarget(tgt)
+    other.setTargetNormals(got)
+    for h in (icp, other):
+        h.setMaxCorrespondenceDistance(0.5)
+        h.setMaximumIterations(1)   # (further ones end at the same pose with any normals)
+        h.align()
+    T = icp.getFinalTransformation()
+    assert np.array_equal(T, other.getFinalTransformation(), equal_nan=True)
+    if n < 100:
+        return   # too few points to hold a plane-to-plane pose still to a tolerance
+    p = oracle.params(max_iter=1, r_max=0.5, mode=1, anchor=icp.getAnchor())
+    plain = oracle.icp(src, tgt, p, tgt_normals=got)
+    assert plain["n_corr"] == icp.getResult()["n_corr"] and np.abs(T - plain["T"]).max() < 1e-5
+    moved = oracle.icp(src, tgt, p, tgt_normals=np.roll(got, 1, axis=0))
+    assert np.abs(T - moved["T"]).max() > 1e-4
 
 
 @pytest.mark.parametrize("k", [7, 20])
