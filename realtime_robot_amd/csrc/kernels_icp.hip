@@ -254,8 +254,7 @@ struct GlobalVis {
     }
   }
   // D (4 or 8) independent loads in flight per step: the gathers are
-  // latency-bound, and the deeper variant needs the registers of a kernel
-  // that runs 2 waves per SIMD.  A step always takes D neighbouring slots, one
+  // latency-bound (which kernel takes which D: see k_icp).  A step always takes D neighbouring slots, one
   // address and D offsets, whatever is left of the range (moved back at the
   // target's end, for targets of at least D points): points beyond the range
   // are points of the target all the same, and a short range costs one round
@@ -1053,7 +1052,11 @@ __global__ __launch_bounds__(kBlock, WAVES) void k_icp(DevEngine e) {
 // and the seeds' points.  The transform is read with agent-scope loads and no
 // acquire: nothing else written during the launch is read by the search (its
 // seeds are the workgroup's own), so the target's cells stay in the L1 from
-// iteration to iteration.  A whole call on 2k x 10k points 1.70 -> 0.92 ms and
+// iteration to iteration.  That rests on the machine, not on the language's
+// model: the solving workgroup's release writes the transform back before the
+// generation word; these loads are issued after the word's value has arrived (a
+// branch on it, and a fence that the compiler may not move them over) and, being
+// agent-scope, pass the L1 and see what the other XCDs wrote back.  A whole call on 2k x 10k points 1.70 -> 0.92 ms and
 // on 10k x 20k 2.23 -> 1.22 ms (38 -> 18 us an iteration, of which the sums and
 // the solve take 6); 30k x 366k points point-to-plane: the launch 1.0 -> 0.7 ms.
 //
@@ -1210,6 +1213,7 @@ __global__ __launch_bounds__(kBlock, 2) void k_icp_one(DevEngine e) {
             wv = load_relaxed(word);
           }
           const bool run = !(wv & kFinishedBit) && (int)wv == pass;
+          __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");  // no instruction: an order for the compiler
           if (run && lane < 12) sh.m[lane] = (float)load_relaxed(&e.st[0].T[(lane & 3) * 4 + (lane >> 2)]);
           if (lane == 0) {
             sh.run = run ? 1 : 0;
