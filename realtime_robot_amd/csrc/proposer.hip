@@ -75,8 +75,9 @@ struct ParamLayout {
 // GEMM: C[M x N] = op(A)[M x K] * op(B)[K x N] (+ bias[N]) (ReLU)
 //   A(i,k) = ta ? A[k*lda + i] : A[i*lda + k]   (bf16)
 //   B(k,j) = tb ? B[j*ldb + k] : B[k*ldb + j]   (bf16)
-// Output FP32 (atomicAdd when split-K) or BF16.  64 x 64 tile per workgroup
-// (2 x 2 waves of 32 x 32 MFMA tiles), K staged through LDS 64 at a time.
+// Output FP32 (atomicAdd when split-K, which rtr_gemm_bf16 alone asks for) or BF16.
+// 64 x 64 tile per workgroup (2 x 2 waves of 32 x 32 MFMA tiles), K staged
+// through LDS 64 at a time.
 // ---------------------------------------------------------------------------
 struct GemmArgs {
   const uint16_t* A;
